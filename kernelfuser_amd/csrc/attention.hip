@@ -1,13 +1,11 @@
-// The general attention kernel (attn_fwd_kernel: any D in {128, 256} and
-// GQA ratio, 4 waves = 128 query rows of one head, GEMM1 of tile t+1 issued
-// ahead of the softmax and GEMM2 of tile t, lean online softmax with an exact
-// redo, split-KV halves at D = 256) and the dispatch of launch_attention over
-// the three kernels.  Counterpart of the reference's attention_v2_kernel
-// (src/e1_rope_publication_v1.py:608-649) and factored_attention_kernel
-// (src/e1_qk_publication_v3.py:612-638).  The arithmetic the kernels share
-// (Q prologue, online softmax, MFMA operand layouts, LDS staging, epilogue) is
-// in attn_common.h; the ping-pong kernel is in attn_pp.hip, the wide-wave
-// kernel in attn_wide.hip.
+// The dispatch of launch_attention over the attention kernels, and the general
+// kernel's mode 'full' (K normalised tile by tile).  Counterpart of the
+// reference's attention_v2_kernel (src/e1_rope_publication_v1.py:608-649) and
+// factored_attention_kernel (src/e1_qk_publication_v3.py:612-638).  The
+// arithmetic the kernels share (Q prologue, online softmax, MFMA operand
+// layouts, LDS staging, epilogue) is in attn_common.h; the general kernel's
+// other modes are in attn_fwd.h, the ping-pong kernel in attn_pp.hip, the
+// wide-wave kernel in attn_wide.hip.
 #include <math.h>
 
 #include <atomic>
@@ -16,17 +14,19 @@
 #include <string>
 
 #include "attn_common.h"
+#include "attn_split.h"
 
 namespace kfmi {
 namespace {
 
 // ---------------------------------------------------------------------------
-// General kernel: one head, 4 waves x 32 rows, D in {128, 256}.
+// Mode 'full': K arrives raw and every tile gets the K prologue (FK).  One head,
+// 4 waves x 32 rows, GEMM1 of tile t+1 issued ahead of the softmax and GEMM2 of
+// tile t, exact online softmax.
 // ---------------------------------------------------------------------------
-template <int D, int BN, bool CAUSAL, int PRO, int ST, bool FK = false>
+template <int D, int BN, bool CAUSAL, int PRO, int ST, bool FK>
 __global__ __launch_bounds__(256, (D == 128 ? 2 : 1)) void attn_fwd_kernel(AttnParams p) {
-  // FK: K arrives raw and every tile gets the K prologue of mode 'full'.
-  static_assert(!FK || PRO == PRO_NORM || PRO == PRO_NORM_ROPE, "mode 'full' fuses Q as well");
+  static_assert(FK && (PRO == PRO_NORM || PRO == PRO_NORM_ROPE), "the other forms: attn_fwd.h");
   constexpr int BM = 128;            // query rows per workgroup (4 waves x 32)
   constexpr int RB = 2 * D;          // bytes per K/V row
   constexpr int TILE = BN * RB;      // bytes per K or V tile
@@ -39,14 +39,9 @@ __global__ __launch_bounds__(256, (D == 128 ? 2 : 1)) void attn_fwd_kernel(AttnP
   __shared__ __attribute__((aligned(1024))) unsigned char smem[4 * TILE];
 
   clock_stamp<false>(p.stamps);
-  // Two-slot pairing (slot2 > 0): the second slot holds the short causal
-  // blocks, whose workgroups have slack; they start about 12k cycles late, so
-  // the long blocks of the first slot, which set the kernel's end, stage their
-  // tables, Q rows and first tiles without that traffic.  Measured against no
-  // delay, alternated on one box: B=1 S=2048 46.5 vs 47.5 us, S=1536 33.6 vs
-  // 33.9 us, B=2 S=1024 28.1 vs 28.7 us; 6k cycles gained less at S=2048
-  // (46.8 us), 18k cycles lost at B=2 S=1024 (28.8 us).  (s_sleep n waits
-  // about 64n cycles.)
+  // Two-slot pairing (slot2 > 0): the short causal blocks of the second slot
+  // start about 12k cycles late (s_sleep n waits about 64n cycles), so the long
+  // blocks of the first, which set the kernel's end, load without that traffic.
   if (CAUSAL && p.slot2 > 0 && (int)blockIdx.x >= p.slot2) {
     __builtin_amdgcn_s_sleep(96);
     __builtin_amdgcn_s_sleep(96);
@@ -137,55 +132,20 @@ __global__ __launch_bounds__(256, (D == 128 ? 2 : 1)) void attn_fwd_kernel(AttnP
     copy_v(t0, V0);
     if (t0 + 1 < nT) copy_k(t0 + 1, K1);
   };
-  // D = 128 with RoPE: the rotary-table rows of the wave's 32 positions are
-  // first staged in the K/V buffers (cos in the first 32 KiB, sin in the
-  // second) with coalesced copies (8 per table per wave, the K tiles' chunk
-  // swizzle, so kra[c] addresses the lane's chunks) instead of loads that
-  // each touch 32 rows.  Once every wave holds its rows in registers the
-  // first K/V copies are issued; they land while the prologue computes.
-  constexpr bool STAGE_TAB = D == 128 && PRO == PRO_NORM_ROPE && !FK;
-  StagedTables tab;
-  if constexpr (STAGE_TAB) {
-    const i32x4_t crs = buffer_rsrc(p.cos, (uint32_t)(S * RB));
-    const i32x4_t srs = buffer_rsrc(p.sin, (uint32_t)(S * RB));
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int j = 8 * w + i;  // rows 4j .. 4j+3 of the block
-      const uint32_t voff = copy_lane_offset<D>(j, lane, false) + (uint32_t)(qb * BM * RB);
-      copy16_to_lds(crs, lds0 + j * 1024, voff);
-      copy16_to_lds(srs, lds0 + 32768 + j * 1024, voff);
-    }
-    tab.cos = smem + w * 32 * RB;
-    tab.sin = tab.cos + 32768;
-    tab.off = kra;
-  } else {
-    // Start the first copies before the prologue's own global loads.
-    first_copies();
-  }
-
+  // Start the first copies before the prologue's own global loads.
+  first_copies();
   bf16x8_t qreg[NC];
   float cl;
-  if constexpr (STAGE_TAB) {
-    q_prologue<D, PRO, ST, false, true>(p, qoff, qrow, qvalid, g, qreg, cl, tab, [&]() {
-      __syncthreads();  // every wave's table reads have completed
-      first_copies();
-    });
-  } else {
-    q_prologue<D, PRO, ST>(p, qoff, qrow, qvalid, g, qreg, cl);
-  }
+  q_prologue<D, PRO, ST>(p, qoff, qrow, qvalid, g, qreg, cl);
 
   f32x16_t o[NDB];
   Softmax<D, BN, CAUSAL> sm;
-  bool bad = false;  // a lean tile of this lane failed its overflow guard
 
   // Pipeline (one barrier per KV tile): iteration t issues the copies of
   // K(t+2) and V(t+1), then GEMM1 of tile t+1 and the softmax + GEMM2 of tile
-  // t; each copy has a full iteration to land.  PAR = t % 2 selects buffers;
-  // LEAN selects Softmax::step_lean (hot path) or Softmax::step (exact).
-  auto iteration = [&](auto par, auto lean, auto first, int t, f32x16_t (&cur)[NKB], f32x16_t (&nxt)[NKB]) {
+  // t; each copy has a full iteration to land.  PAR = t % 2 selects buffers.
+  auto iteration = [&](auto par, int t, f32x16_t (&cur)[NKB], f32x16_t (&nxt)[NKB]) {
     constexpr int PAR = decltype(par)::value;
-    constexpr bool LEAN = decltype(lean)::value;
-    constexpr bool FIRST = decltype(first)::value;
     constexpr int KNEXT = PAR ? K0 : K1;   // holds K(t+1)
     constexpr int KFREE = PAR ? K1 : K0;   // held K(t), read in the previous iteration
     constexpr int VCUR = PAR ? V1 : V0;    // holds V(t)
@@ -195,144 +155,33 @@ __global__ __launch_bounds__(256, (D == 128 ? 2 : 1)) void attn_fwd_kernel(AttnP
     if (t + 2 < nT) copy_k(t + 2, KFREE);
     if (t + 1 < nT) copy_v(t + 1, VFREE);
     if (t + 1 < nTw) {
-      if constexpr (FK)
-        gemm1_fused_k<D, BN, ST, PRO == PRO_NORM_ROPE>(smem, KNEXT, kra, qreg, nxt, p, (t + 1) * BN, g, lr);
-      else
-        gemm1<D, BN>(smem, KNEXT, kra, qreg, nxt);
+      gemm1_fused_k<D, BN, ST, PRO == PRO_NORM_ROPE>(smem, KNEXT, kra, qreg, nxt, p, (t + 1) * BN, g, lr);
     }
     if (t < nTw) {
       bf16x8_t pb[NK16];
-      if constexpr (LEAN)
-        sm.template step_lean<FIRST>(cur, t, q0, qrow, S, g, cl, pb, bad);
-      else
-        sm.step(cur, t, q0, qrow, S, g, cl, o, pb);
+      sm.step(cur, t, q0, qrow, S, g, cl, o, pb);
       gemm2<D, BN>(smem, VCUR, vra, pb, o);
     }
   };
-  // One sweep over the work item's KV tiles; the first K/V copies must have
-  // been issued.
-  auto sweep = [&](auto lean) {
 #pragma unroll
-    for (int db = 0; db < NDB; ++db) o[db] = f32x16_t{};
-    sm = Softmax<D, BN, CAUSAL>{};
-    f32x16_t sa[NKB], sb[NKB];
-    wait_copies();
-    __syncthreads();
-    if (t0 < nTw) {
-      if constexpr (FK)
-        gemm1_fused_k<D, BN, ST, PRO == PRO_NORM_ROPE>(smem, K0, kra, qreg, sa, p, t0 * BN, g, lr);
-      else
-        gemm1<D, BN>(smem, K0, kra, qreg, sa);
-    }
-    // the first tile is peeled (it alone reduces the row max on the lean path)
-    iteration(std::integral_constant<int, 0>{}, lean, std::true_type{}, t0, sa, sb);
-    for (int t = t0 + 1; t < nT;) {
-      iteration(std::integral_constant<int, 1>{}, lean, std::false_type{}, t, sb, sa);
-      if (++t >= nT) break;
-      iteration(std::integral_constant<int, 0>{}, lean, std::false_type{}, t, sa, sb);
-      ++t;
-    }
-  };
-  if constexpr (FK) {
-    sweep(std::false_type{});  // mode 'full' runs at the register limit: exact path only
-  } else {
-    sweep(std::true_type{});
-    // Probabilities up to 2^64 keep the row sums finite but can still
-    // overflow O when |V| is large.
-    bad |= any_not_finite(o);  // no short circuit: a branch here costs the loop registers
-    // A lean tile failed somewhere in the workgroup (a logit far above the
-    // first tile's row max, or an accumulator that overflowed): every wave
-    // redoes the item on the exact path.
-    if (__syncthreads_or(bad)) {
-      first_copies();
-      sweep(std::false_type{});
-    }
+  for (int db = 0; db < NDB; ++db) o[db] = f32x16_t{};
+  f32x16_t sa[NKB], sb[NKB];
+  wait_copies();
+  __syncthreads();
+  if (t0 < nTw) gemm1_fused_k<D, BN, ST, PRO == PRO_NORM_ROPE>(smem, K0, kra, qreg, sa, p, t0 * BN, g, lr);
+  for (int t = t0; t < nT;) {
+    iteration(std::integral_constant<int, 0>{}, t, sa, sb);
+    if (++t >= nT) break;
+    iteration(std::integral_constant<int, 1>{}, t, sb, sa);
+    ++t;
   }
 
-  // the host plans splits for D = 256 only (plan_split)
-  if (D != 256 || sid < 0) {
-    if constexpr (FK) {
-      // mode 'full' runs at the register limit: direct stores
-      store_rows<D>(p.out + qoff * D, qrow, qvalid, g, sm.l_run, o);
-    } else {
-      __syncthreads();  // the K/V buffers become the epilogue's staging tiles
-      store_rows_lds<D>(smem + w * (32 * 2 * D), p.out + qoff * D, q0, S, lane, sm.l_run, o);
-    }
-    clock_stamp<true>(p.stamps);
-    return;
-  }
-  // ---- one half of a split query block: publish the partial state (O
-  // relative to m_run, the lane's row-sum share, m_run); the half that
-  // finishes second reads the other's, merges and stores, and re-arms the
-  // counter.  Slot layout (floats): O quad q of thread tid at
-  // [(q * 256 + tid) * 4], m_run at [NQ * 1024 + tid], l_run after it.
-  //
-  // The slots are written and read with agent-coherent accesses (cache
-  // policy SC1, what the compiler gives agent-scope atomic accesses on
-  // gfx950): a store that has completed (vmcnt) is visible to SC1 loads on
-  // any XCD.  That orders the handover through the counter without the L2
-  // writeback and invalidate that a device-scope fence costs.
-  constexpr int NQ = NDB * 4;
-  constexpr int SLOT = (NQ * 4 + 2) * 256;  // floats
-  constexpr int SC1 = 16;
-  const int part = t0 > 0 ? 1 : 0;
-  // wave-uniform (sid, b, h are per workgroup): keeps the descriptors in SGPRs
-  const int pair = __builtin_amdgcn_readfirstlane(sid * nbh + (b * p.Hq + h));
-  const auto mine =
-      __builtin_amdgcn_make_buffer_rsrc(p.partials + (int64_t)(2 * pair + part) * SLOT, 0, SLOT * 4, 0x00020000);
-  const auto other =
-      __builtin_amdgcn_make_buffer_rsrc(p.partials + (int64_t)(2 * pair + 1 - part) * SLOT, 0, SLOT * 4, 0x00020000);
-#pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    const f32x4_t v = {o[q / 4][(q % 4) * 4], o[q / 4][(q % 4) * 4 + 1], o[q / 4][(q % 4) * 4 + 2],
-                       o[q / 4][(q % 4) * 4 + 3]};
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), mine, (q * 256 + tid) * 16, 0, SC1);
-  }
-  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, sm.m_run), mine, (NQ * 1024 + tid) * 4, 0, SC1);
-  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, sm.l_run), mine, (NQ * 1024 + 256 + tid) * 4, 0,
-                                        SC1);
-  wait_copies();  // every store of this thread has completed
-  __syncthreads();
-  __shared__ int arrived_before;
-  if (tid == 0) {
-    // Release/acquire at agent scope around the arrival counter (the
-    // memory model's own mapping: L2 writeback before, invalidate after), so
-    // the handover is ordered even where the SC1 accesses alone would not
-    // be; one thread per workgroup, after the barrier that follows every
-    // thread's completed stores.
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    arrived_before = atomicAdd(p.counters + pair, 1);
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  }
-  __syncthreads();
-  if (arrived_before == 0) {  // the other half merges
-    clock_stamp<true>(p.stamps);
-    return;
-  }
-  // Merge in fixed (first half, second half) operand order, whichever half
-  // runs it, with explicit fmaf, so the result does not depend on timing.
-  const float mo = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(other, (NQ * 1024 + tid) * 4, 0, SC1));
-  const float lo =
-      __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(other, (NQ * 1024 + 256 + tid) * 4, 0, SC1));
-  const float m0 = part == 0 ? sm.m_run : mo, m1 = part == 0 ? mo : sm.m_run;
-  const float m = fmaxf(m0, m1);
-  // rows past S may hold -inf maxima in both halves; they are not stored
-  const float a0 = m0 == m ? 1.0f : __builtin_amdgcn_exp2f(m0 - m);
-  const float a1 = m1 == m ? 1.0f : __builtin_amdgcn_exp2f(m1 - m);
-#pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    const f32x4_t v = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(other, (q * 256 + tid) * 16, 0, SC1));
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const float r = o[q / 4][(q % 4) * 4 + k];
-      const float x0 = part == 0 ? r : v[k], x1 = part == 0 ? v[k] : r;
-      o[q / 4][(q % 4) * 4 + k] = fmaf(x0, a0, x1 * a1);
-    }
-  }
-  const float l0 = part == 0 ? sm.l_run : lo, l1 = part == 0 ? lo : sm.l_run;
-  __syncthreads();
-  store_rows_lds<D>(smem + w * (32 * 2 * D), p.out + qoff * D, q0, S, lane, fmaf(l0, a0, l1 * a1), o);
-  if (tid == 0) atomicExch(p.counters + pair, 0);
+  // direct stores (the kernel runs at the register limit); the host plans
+  // splits for D = 256 only (plan_split)
+  if (D != 256 || sid < 0) store_rows<D>(p.out + qoff * D, qrow, qvalid, g, sm.l_run, o);
+  else
+    split_finish<D>(p, smem + w * (32 * 2 * D), sid * nbh + (b * p.Hq + h), t0 > 0 ? 1 : 0, qoff, q0, tid, lane, sm.m_run,
+                    sm.l_run, o);
   clock_stamp<true>(p.stamps);
 }
 
@@ -359,10 +208,8 @@ hipError_t launch_t(const AttnParams &p, int kind, int blocks, hipStream_t s) {
     if (kind == KFMI_KERNEL_WIDE) return launch_wide(p, CAUSAL, PRO, ST, blocks, s);
     if (kind == KFMI_KERNEL_PINGPONG) return launch_pp(p, CAUSAL, PRO, ST, blocks, s);
   }
-  hipLaunchKernelGGL((attn_fwd_kernel<D, BN, CAUSAL, PRO, ST>), dim3(blocks), dim3(256), 0, s, p);
-  launch_log_add(reinterpret_cast<const void *>(&attn_fwd_kernel<D, BN, CAUSAL, PRO, ST, false>),
-                 fwd_name<D, BN, CAUSAL, PRO, ST, false>(), blocks, 256);
-  return hipGetLastError();
+  if constexpr (D == 256) return launch_fwd256(p, CAUSAL, PRO, ST, blocks, s);
+  else return launch_fwd128(p, CAUSAL, PRO, ST, blocks, s);
 }
 
 template <int D, int BN, bool CAUSAL>
@@ -591,6 +438,10 @@ hipError_t launch_attention(const AttnArgs &a, hipStream_t stream) {
   p.S = a.S;
   p.B = (int)a.B; p.Hq = (int)a.Hq; p.Hkv = (int)a.Hkv;
   p.eps = a.eps;
+  p.by_nbh = FastDiv::of((uint32_t)(a.B * a.Hq));
+  p.by_hq = FastDiv::of((uint32_t)a.Hq);
+  p.by_hkv = FastDiv::of((uint32_t)a.Hkv);
+  p.by_g = FastDiv::of((uint32_t)(a.Hq / a.Hkv));
   const bool factored = a.prologue == PRO_FACTORED_READ || a.prologue == PRO_FACTORED_CALC;
   // rope:636 SCALE*log2e; qk:621 D**-.5*log2e (both formed in double, then FP32)
   p.c_scale = (float)((factored ? 1.0 / sqrt((double)a.D) : a.scale) * LOG2E);

@@ -22,8 +22,9 @@
 //                    the other computes exponentials.  Each K/V tile staged in
 //                    LDS serves every head of the workgroup.
 //   attn_fwd_kernel  any D in {128, 256} and GQA ratio: 4 waves = 128 query
-//                    rows of one head; GEMM1 of tile t+1 is issued ahead of the
-//                    softmax and GEMM2 of tile t.
+//                    rows of one head; every wave pipelines GEMM1, softmax and
+//                    GEMM2 of consecutive key blocks inside itself
+//                    (attn_fwd.h; mode 'full': attention.hip, phase by phase).
 //   attn_ww_kernel   D=128, Hq/Hkv a multiple of 4, on request only: 4 waves,
 //                    one per SIMD, each holding 64 query rows of one head and
 //                    pipelining GEMM1, softmax and GEMM2 of consecutive tiles
@@ -87,6 +88,23 @@
 
 namespace kfmi {
 
+// n / d for n < 2^31 by one multiplication (round-up reciprocal of 31 + ceil(log2
+// d) bits); mul = 0 stands for d = 1.  A division of uniform values costs the
+// scalar-vector round trips of a floating-point reciprocal, ~150 cycles each,
+// at a workgroup's start.
+struct FastDiv {
+  uint32_t mul, shift, mask;
+  __host__ static FastDiv of(uint32_t d) {
+    uint32_t l = 0;
+    while (((uint64_t)1 << l) < d) ++l;
+    if (l == 0) return {0u, 0u, ~0u};
+    return {(uint32_t)((((uint64_t)1 << (31 + l)) + d - 1) / d), l - 1, 0u};
+  }
+  __device__ __forceinline__ int div(int n) const {
+    return (int)((__umulhi((uint32_t)n, mul) >> shift) + ((uint32_t)n & mask));
+  }
+};
+
 struct AttnParams {
   const uint16_t *q, *k, *v, *gq, *cos, *sin;
   const uint16_t *gk;  // K's gamma for the per-tile K prologue (mode 'full'), else NULL
@@ -106,6 +124,7 @@ struct AttnParams {
   // slot takes the query blocks shortest first and each CU's pair sums to
   // the same number of key tiles
   int slot2;
+  FastDiv by_nbh, by_hq, by_hkv, by_g;  // general kernel: B*Hq, Hq, Hkv, Hq/Hkv
   float c_scale;  // scale*log2(e); for the factored prologues D^-1/2*log2(e)
   float eps;
   // Split-KV plan of the general kernel (n_items > 0): work item r of the
@@ -160,6 +179,34 @@ __device__ __forceinline__ float rope_elem(float n, float np, float c, float s, 
   return first ? p0 - p1 : p0 + p1;
 }
 
+// The HF and legacy chains over the eight columns of a chunk, rounding two
+// values at a time (one conversion and two unpacks a pair instead of two and
+// two): VALU time that nothing hides on a workgroup's first item.
+__device__ __forceinline__ void round8(float (&x)[8]) { unpack8(pack8(x), x); }
+template <int ST>
+__device__ __forceinline__ void norm8(const float (&x)[8], float inv, const float (&g)[8], float (&n)[8]) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) n[j] = __fmul_rn(x[j], inv);
+  if constexpr (ST == ST_HF) round8(n);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) n[j] = __fmul_rn(n[j], g[j]);
+  round8(n);
+}
+template <int ST>
+__device__ __forceinline__ void rope8(const float (&n)[8], const float (&np)[8], const float (&c)[8],
+                                      const float (&s)[8], bool first, float (&y)[8]) {
+  float p0[8], p1[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    p0[j] = __fmul_rn(n[j], c[j]);
+    p1[j] = __fmul_rn(np[j], s[j]);
+  }
+  round8(p0);
+  round8(p1);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) y[j] = first ? p0[j] - p1[j] : p0[j] + p1[j];
+}
+
 __device__ __forceinline__ bf16x8_t as_bf16x8(const u32x4_t &w) { return __builtin_bit_cast(bf16x8_t, w); }
 
 typedef int i32x4_t __attribute__((ext_vector_type(4)));
@@ -199,11 +246,6 @@ __device__ __forceinline__ void copy16_to_lds(const i32x4_t &rsrc, uint32_t lds,
 __device__ __forceinline__ void wait_copies() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 constexpr float RESCALE_SLACK = 8.0f;  // log2 units: probabilities stay <= 2^8
-// Lean-softmax guard: a lane's partial sum of one tile's probabilities must
-// stay below 2^64, so every probability does and O accumulates far inside
-// FP32 range; otherwise the work item is redone with the exact softmax.
-constexpr float FAST_LIMIT = 0x1p64f;
-
 // Phase fences: an empty volatile asm that takes the phase's results as
 // inputs, so the compiler finishes computing them before the barrier that
 // ends the phase instead of sinking that work into the next phase.
@@ -380,10 +422,15 @@ __device__ __forceinline__ void q_prologue(const AttnParams &p, int64_t qoff, in
         unpack8(raw[c2], x2);
         unpack8(graw[c], g1);
         unpack8(graw[c2], g2);
+        if constexpr (ST == ST_FP32) {  // no intermediate rounding
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          n1[j] = norm_elem<ST>(x1[j], inv, g1[j]);
-          n2[j] = norm_elem<ST>(x2[j], inv, g2[j]);
+          for (int j = 0; j < 8; ++j) {
+            n1[j] = norm_elem<ST>(x1[j], inv, g1[j]);
+            n2[j] = norm_elem<ST>(x2[j], inv, g2[j]);
+          }
+        } else {
+          norm8<ST>(x1, inv, g1, n1);
+          norm8<ST>(x2, inv, g2, n2);
         }
         if constexpr (PRO == PRO_NORM_ROPE) {
           float cs1[8], sn1[8], cs2[8], sn2[8];
@@ -391,10 +438,15 @@ __device__ __forceinline__ void q_prologue(const AttnParams &p, int64_t qoff, in
           unpack8(sraw[c], sn1);
           unpack8(craw[c2], cs2);
           unpack8(sraw[c2], sn2);
+          if constexpr (ST == ST_FP32) {
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            y1[j] = rope_elem<ST>(n1[j], n2[j], cs1[j], sn1[j], true);
-            y2[j] = rope_elem<ST>(n2[j], n1[j], cs2[j], sn2[j], false);
+            for (int j = 0; j < 8; ++j) {
+              y1[j] = rope_elem<ST>(n1[j], n2[j], cs1[j], sn1[j], true);
+              y2[j] = rope_elem<ST>(n2[j], n1[j], cs2[j], sn2[j], false);
+            }
+          } else {
+            rope8<ST>(n1, n2, cs1, sn1, true, y1);
+            rope8<ST>(n2, n1, cs2, sn2, false, y2);
           }
         } else {
 #pragma unroll
@@ -428,7 +480,7 @@ struct Softmax {
   static constexpr int NKB = BN / 32, NK16 = BN / 16, NDB = D / 32;
   float m_run = FOLD ? 0.f : -INFINITY;  // reference max of logits (log2 domain)
   float l_run = 0.f;                     // this lane's partial row sum
-  bool started = false;                  // a tile has set m_run (FOLD and step_lean)
+  bool started = false;                  // a tile has set m_run (FOLD)
 
   // GEMM1 accumulator start value of this lane (FOLD: -m_run).
   __device__ __forceinline__ float acc_init() const { return FOLD ? -m_run : 0.f; }
@@ -516,68 +568,6 @@ struct Softmax {
     pack(s, pb);
   }
 
-  // Lean tile (the general kernel's hot path).  The first tile of a sweep
-  // (FIRST, peeled by the caller so later tiles carry no branch) sets m_run
-  // to the tile's exact row max (O and l are still zero, so nothing is
-  // rescaled); every later tile takes p = exp2(logit - m_run)
-  // with no max reduction and no rescale.  That is the same softmax (one
-  // constant shift per row), valid as long as no probability overflows:
-  // a lane whose partial tile sum is not below FAST_LIMIT sets `bad` (rows
-  // at or past S excluded), and the caller then redoes the whole work item
-  // with step().  O never changes here, which keeps this path's register
-  // footprint at that of the accumulators alone.
-  template <bool FIRST>
-  __device__ __forceinline__ void step_lean(f32x16_t (&s)[NKB], int t, int q0, int qrow, int64_t S, int g, float cl,
-                                            bf16x8_t (&pb)[NK16], bool &bad) {
-    const int kt = t * BN;
-    const bool need_mask = (CAUSAL && kt + BN - 1 > q0) || (kt + BN > S);
-    if (need_mask) {
-      const int last = (int)(S - 1);
-      const int lim = (CAUSAL ? (qrow < last ? qrow : last) : last) - kt - 4 * g;
-#pragma unroll
-      for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-          if (32 * kb + 8 * (i >> 2) + (i & 3) > lim) s[kb][i] = -INFINITY;
-    }
-    if constexpr (FIRST) {
-      float mt[NKB * 8];
-#pragma unroll
-      for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) mt[kb * 8 + i] = fmaxf(s[kb][2 * i], s[kb][2 * i + 1]);
-#pragma unroll
-      for (int n = NKB * 8; n > 1; n = (n + 1) / 2)
-#pragma unroll
-        for (int i = 0; i + (n + 1) / 2 < n; ++i) mt[i] = fmaxf(mt[i], mt[i + (n + 1) / 2]);
-      const float mx = max_halves(mt[0]);
-      if constexpr (FOLD) {
-        m_run += mx;  // scores held logit - m_run with m_run = 0
-#pragma unroll
-        for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) s[kb][i] -= mx;
-      } else {
-        m_run = mx * cl;
-      }
-      started = true;
-    }
-    float ls[4] = {0.f, 0.f, 0.f, 0.f};
-    const float nm = -m_run;
-#pragma unroll
-    for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float pv = FOLD ? __builtin_amdgcn_exp2f(s[kb][i]) : __builtin_amdgcn_exp2f(__builtin_fmaf(s[kb][i], cl, nm));
-        s[kb][i] = pv;
-        ls[i & 3] += pv;
-      }
-    const float lt = (ls[0] + ls[1]) + (ls[2] + ls[3]);
-    l_run += lt;
-    bad |= qrow < S && !(lt < FAST_LIMIT);
-    pack(s, pb);
-  }
-
   // P^T operands: 16-key step c2 <- registers 8*(c2%2) .. +7 of block c2/2
   // (registers 4q..4q+3 of a block hold keys 8q + 4*g + 0..3).
   __device__ __forceinline__ void pack(const f32x16_t (&s)[NKB], bf16x8_t (&pb)[NK16]) const {
@@ -602,33 +592,6 @@ struct Softmax {
     }
   }
 };
-
-// GEMM1: S^T (BN keys x 32 queries) of the K tile at LDS byte kbuf.
-constexpr int G1_AHEAD = 2;
-template <int D, int BN>
-__device__ __forceinline__ void gemm1(const unsigned char *smem, int kbuf, const uint32_t (&kra)[8],
-                                      const bf16x8_t (&qreg)[D / 16], f32x16_t (&s)[BN / 32]) {
-  constexpr int RB = 2 * D, NKB = BN / 32, NC = D / 16;
-#pragma unroll
-  for (int kb = 0; kb < NKB; ++kb) s[kb] = f32x16_t{};
-#pragma unroll
-  for (int c = 0; c < NC; ++c) {  // alternating accumulation chains
-#pragma unroll
-    for (int kb = 0; kb < NKB; ++kb) {
-      const bf16x8_t a = *reinterpret_cast<const bf16x8_t *>(smem + kbuf + kb * 32 * RB + kra[c & 7] + (c >> 3) * 256);
-      s[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qreg[c], s[kb], 0, 0, 0);
-    }
-  }
-  // Issue order: K reads run G1_AHEAD MFMAs ahead, so an MFMA's operand was
-  // requested several MFMAs (~32 cycles each) before it, past the LDS
-  // latency.
-  __builtin_amdgcn_sched_group_barrier(0x100, G1_AHEAD, 0);
-#pragma unroll
-  for (int i = 0; i < NKB * NC; ++i) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    if (i + G1_AHEAD < NKB * NC) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-  }
-}
 
 // GEMM1 with the K prologue of mode 'full' (rope:630-631, FUSE_K): the lane's
 // raw K row chunks are read from the tile (row 32*kb + lr: columns 16c + 8g ..
@@ -663,7 +626,7 @@ __device__ __forceinline__ void gemm1_fused_k(const unsigned char *smem, int kbu
     const int key = key0 + 32 * kb + lr;
     const int64_t trow = key < p.S ? (int64_t)key * D : 0;
     // pass 2: one rotate-half pair (c, c + D/32 chunks) at a time; the MFMAs
-    // accumulate in chunk order 0 .. NC-1, as in gemm1.
+    // accumulate in chunk order 0 .. NC-1.
     bf16x8_t khi[HC];
     s[kb] = f32x16_t{};
 #pragma unroll
@@ -893,6 +856,8 @@ __device__ __forceinline__ bool any_not_finite(const f32x16_t (&o)[N]) {
 // Launchers of the kernels that live in their own files (runtime dispatch
 // over the template instances of each file).
 hipError_t launch_pp(const AttnParams &p, bool causal, int pro, int st, int blocks, hipStream_t s);
+hipError_t launch_fwd128(const AttnParams &p, bool causal, int pro, int st, int blocks, hipStream_t s);
+hipError_t launch_fwd256(const AttnParams &p, bool causal, int pro, int st, int blocks, hipStream_t s);
 hipError_t launch_wide(const AttnParams &p, bool causal, int pro, int st, int blocks, hipStream_t s);
 
 }  // namespace kfmi

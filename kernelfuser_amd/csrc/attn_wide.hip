@@ -5,6 +5,7 @@
 #include <type_traits>
 
 #include "attn_common.h"
+#include "attn_mfma.h"
 
 namespace kfmi {
 namespace {
@@ -165,36 +166,9 @@ __device__ __forceinline__ void ww_mask(f32x16_t (&s)[2][2], int kt, int q0, int
   }
 }
 
-// v_mfma_f32_32x32x16_bf16 as inline assembly, so that each operand sits in
-// the register file this kernel needs: scores in VGPRs (the VALU reads them),
-// O and the Q operands in AGPRs.  (With the builtin the compiler puts every
-// accumulator of a kernel in one file, and O plus two score buffers do not
-// fit in the 256 AGPRs.)  The compiler does not know these are MFMAs, so the
-// kernel keeps their dependency distances itself.  For this MFMA on gfx950
-// the compiler's own hazard rules are: none for an accumulation chain on one
-// register, 2 wait states from a VALU write to an MFMA operand read, 12 from
-// an MFMA result to any other instruction that reads it (and an MFMA source
-// register may be overwritten right after issue).  The loop below consumes
-// every MFMA result, and feeds every VALU result to an MFMA, at least eight
-// MFMAs later; everywhere else an explicit wait (mfma_settle, s_nop) pads the
-// gap, on operands that tie the waiting to the registers concerned.
-__device__ __forceinline__ void mfma_v(f32x16_t &d, const bf16x8_t &a, const bf16x8_t &b) {
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(a), "a"(b));
-}
-__device__ __forceinline__ void mfma_v_from(f32x16_t &d, const bf16x8_t &a, const bf16x8_t &b, const f32x16_t &c) {
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %3" : "=&v"(d) : "v"(a), "a"(b), "v"(c));
-}
-__device__ __forceinline__ void mfma_v_zero(f32x16_t &d, const bf16x8_t &a, const bf16x8_t &b) {
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(d) : "v"(a), "a"(b));
-}
-__device__ __forceinline__ void mfma_a(f32x16_t &d, const bf16x8_t &a, const bf16x8_t &b) {
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(d) : "v"(a), "v"(b));
-}
-// 16 wait states after the last MFMA writing these registers, before any
-// other instruction reads them.
-__device__ __forceinline__ void mfma_settle(f32x16_t (&s)[2][2]) {
-  asm volatile("s_nop 7\n\ts_nop 7" : "+v"(s[0][0]), "+v"(s[0][1]), "+v"(s[1][0]), "+v"(s[1][1]));
-}
+// MFMAs as inline assembly (attn_mfma.h).  The loop below consumes every MFMA
+// result, and feeds every VALU result to an MFMA, at least eight MFMAs later;
+// everywhere else an explicit wait (mfma_settle, s_nop) pads the gap.
 __device__ __forceinline__ void mfma_settle_acc(f32x16_t (&o)[2][4]) {
   asm volatile("s_nop 7\n\ts_nop 7"
                : "+a"(o[0][0]), "+a"(o[0][1]), "+a"(o[0][2]), "+a"(o[0][3]), "+a"(o[1][0]), "+a"(o[1][1]),
@@ -221,14 +195,6 @@ __device__ __forceinline__ void valu_settle(bf16x8_t (&px)[2][4]) {
   asm volatile("s_nop 1"
                : "+v"(px[0][0]), "+v"(px[0][1]), "+v"(px[0][2]), "+v"(px[0][3]), "+v"(px[1][0]), "+v"(px[1][1]),
                  "+v"(px[1][2]), "+v"(px[1][3]));
-}
-
-template <int B, int E, typename F>
-__device__ __forceinline__ void static_for(F &&f) {
-  if constexpr (B < E) {
-    f(std::integral_constant<int, B>{});
-    static_for<B + 1, E>(f);
-  }
 }
 
 template <bool CAUSAL, int PRO, int ST>

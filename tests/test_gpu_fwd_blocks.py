@@ -1,0 +1,87 @@
+"""The general attention kernel at the sizes where its block pipeline can go
+wrong: one to ten 32-key blocks (the K/V rings of two and four tiles wrap, a
+sweep ends on either buffer and either half of a 64-key tile), ragged last
+blocks and rows, waves with no block at all, and both causal modes, for every
+way Q reaches the matrix cores (prepared, normalised, rotated, factored).
+Whole output against the FP32 oracle; and the exact redo of the same shapes,
+started by one key far above the first block's row maximum."""
+import pytest
+import torch
+
+import oracle
+from helpers import announce
+from kernelfuser_amd import (_lib, attention_prefill, factored_attention, make_inputs, prepare_attention,
+                             prepare_factored)
+
+pytestmark = pytest.mark.gpu
+
+# B, S: rows and keys per case
+SIZES = [1, 31, 33, 64, 65, 96, 127, 129, 160, 193, 225, 257, 288, 320]
+
+
+def _expect(xs, causal, rope):
+    q, k, v, gq, gk, cos, sin = (None if t is None else t.cpu() for t in xs.astuple())
+    return oracle.oracle_fp32(q, k, v, gq, gk, cos if rope else None, sin if rope else None, causal)
+
+
+@pytest.mark.parametrize("d", [128, 256])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("path", ["plain", "norm", "rope", "factored"])
+def test_block_counts_whole_output(gpu, d, causal, path):
+    geom = (3, 1, d) if d == 256 else (6, 2, d)
+    for s in SIZES:
+        announce(f"general kernel D={d} S={s} causal={causal} {path}")
+        xs = make_inputs(2, s, geom, 7000 + s, rope=path != "factored").to(gpu)
+        out = torch.full_like(xs.q, float("nan"))
+        kn = torch.empty_like(xs.k)
+        rope = path in ("plain", "rope")
+        with _lib.tuning(attn_kernel="general"):
+            if path == "factored":
+                inv = torch.empty(xs.q.shape[:-1], device=gpu)
+                prepare_factored((xs.q, xs.k, xs.v, xs.gq, xs.gk), inv, kn)
+                factored_attention(xs.q, kn, xs.v, inv, out, causal=causal)
+            else:
+                qn = torch.empty_like(xs.q)
+                prepare_attention(xs.reference7, qn, kn, rope=rope, norm_style="fp32")
+                if path == "plain":
+                    attention_prefill(qn, kn, xs.v, out, causal=causal, fuse_q=False)
+                else:
+                    attention_prefill(xs.q, kn, xs.v, out, gq=xs.gq, cos=xs.cos if rope else None,
+                                      sin=xs.sin if rope else None, causal=causal, norm_style="fp32")
+        torch.cuda.synchronize()
+        gate = oracle.attention_gate(out.cpu(), _expect(xs, causal, rope))
+        assert gate["pass"], (s, gate)
+
+
+@pytest.mark.parametrize("d", [128, 256])
+@pytest.mark.parametrize("where", ["score", "value"])
+def test_redo_whole_output(gpu, d, where):
+    """``score``: the last key's logits lie ~150 (log2) above the first
+    block's, so every row that sees it overflows the shift; ``value``: values
+    near the end of the BF16 range with logits ~20 above, so that only O
+    overflows.  Both leave the lean sweep for the exact softmax."""
+    for s in (40, 65, 130, 290):
+        announce(f"redo D={d} S={s} {where}")
+        g = torch.Generator().manual_seed(s)
+        q = torch.randn((1, 4, s, d), generator=g).bfloat16()
+        k = (0.01 * torch.randn((1, 2, s, d), generator=g)).bfloat16()
+        v = torch.randn((1, 2, s, d), generator=g).bfloat16()
+        # one key along the queries' common direction
+        u = torch.ones(d) / d ** 0.5
+        size = 105.0 if where == "score" else 14.0  # logit = size in natural units: 151 or 20 in log2
+        q += (4.0 * u).bfloat16()
+        k[:, :, s - 1] = (size * d ** 0.5 / 4.0 * u).bfloat16()
+        if where == "value":  # 2^20 * 2^115 overflows FP32, 2^8 (the exact path's slack) * 2^115 does not
+            v = (v.sign() * 2.0 ** 115).bfloat16()
+        out = torch.empty((1, 4, s, d), dtype=torch.bfloat16, device=gpu)
+        qd, kd, vd = q.to(gpu), k.to(gpu), v.to(gpu)
+        with _lib.tuning(attn_kernel="general"):
+            attention_prefill(qd, kd, vd, out, causal=False, fuse_q=False)
+        torch.cuda.synchronize()
+        scale = 2.0 ** -115 if where == "value" else 1.0  # exact in every step
+        w = torch.softmax(torch.matmul(q.double(), k.double().repeat_interleave(2, 1).transpose(2, 3)) * d ** -0.5, -1)
+        ref = torch.matmul(w, v.double().repeat_interleave(2, 1)) * scale
+        got = out.cpu().double() * scale
+        assert bool(torch.isfinite(got).all())
+        # P and O are each rounded to BF16 (2^-9 relative): within 2^-7 of the largest value
+        assert float((got - ref).abs().max()) <= 2.0 ** -7 * float(ref.abs().max()), (s, float((got - ref).abs().max()))
