@@ -345,12 +345,14 @@ namespace {
 // no co-resident workgroup fills the gap).  Blocks with more key tiles than
 // half the maximum are then split into two halves of their key range (the
 // second holds the diagonal), and all items are listed longest first.
-// Measured with the tuning runner: unsplit grids of 64-192 workgroups gain
-// 4-27% (Gemma-3-4B S=2048 57.2 vs 72.6 us), while a grid that already
-// fills every CU (Gemma-3-12B S=2048, 256 workgroups) loses 8% (83.1 vs
-// 77.0 us), so the plan needs fewer query blocks than CUs.  At D = 128 two
-// workgroups share each CU and one already keeps it nearly busy, so the
-// extra prologues of a split cost more than the balance gains.
+// Measured (attention alone, causal, split against unsplit): Gemma-3-4B S=2048
+// 33.6 vs 45.6 us, S=1024 22.2 vs 26.1, S=512 17.3 vs 16.6; a merge costs about
+// 4.5 us, so blocks of up to 8 key tiles stay whole (S=256 14.2 vs 11.6 us).
+// A grid that already fills every CU (Gemma-3-12B S=2048, 256 workgroups) loses
+// by splitting, so the plan needs fewer query blocks than CUs (Gemma-3-12B
+// S=1536, 192 blocks: 36.8 vs 37.8 us).  At D = 128 two workgroups share each
+// CU and one already keeps it nearly busy, so the extra prologues of a split
+// cost more than the balance gains.
 
 // Workspace layout: a counter region of the same size for every shape (one
 // 4-byte arrival counter per split (block, head) pair, at most
@@ -372,6 +374,7 @@ bool plan_split(int64_t B, int64_t Hq, int64_t S, int64_t D, bool causal, int64_
   if (D != 256 || !causal || nqb < 2 || B * Hq * nqb >= cus) return false;
   auto tiles = [&](int64_t qb) { return ((qb + 1) * BM < S ? (qb + 1) * BM : S) + BN - 1; };
   const int64_t t_max = tiles(nqb - 1) / BN;
+  if (t_max <= 8) return false;
   const int64_t half = (t_max + 1) / 2;
   struct Item { int qb, t0, t1, sid; };
   Item items[MAX_SPLIT_ITEMS];

@@ -35,7 +35,7 @@ __device__ __forceinline__ void split_finish(const AttnParams &p, unsigned char 
   for (int q = 0; q < NQ; ++q) {
     const f32x4_t v = {o[q / 4][(q % 4) * 4], o[q / 4][(q % 4) * 4 + 1], o[q / 4][(q % 4) * 4 + 2],
                        o[q / 4][(q % 4) * 4 + 3]};
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), mine, (q * 256 + tid) * 16, 0, SC1);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), mine, tid * 16, q * 4096, SC1);
   }
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, m_run), mine, (NQ * 1024 + tid) * 4, 0, SC1);
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, l_run), mine, (NQ * 1024 + 256 + tid) * 4, 0,
@@ -60,19 +60,35 @@ __device__ __forceinline__ void split_finish(const AttnParams &p, unsigned char 
   const float mo = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(other, (NQ * 1024 + tid) * 4, 0, SC1));
   const float lo =
       __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(other, (NQ * 1024 + 256 + tid) * 4, 0, SC1));
-  const float m0 = part == 0 ? m_run : mo, m1 = part == 0 ? mo : m_run;
-  const float m = fmaxf(m0, m1);
-  // rows past S may hold -inf maxima in both halves; they are not stored
-  const float a0 = m0 == m ? 1.0f : __builtin_amdgcn_exp2f(m0 - m);
-  const float a1 = m1 == m ? 1.0f : __builtin_amdgcn_exp2f(m1 - m);
+  // Every load of a half is issued before the first is waited for (they miss
+  // every cache): left to itself the compiler loads and merges one quad at a
+  // time, 32 round trips.  Gemma-3-4B, B=1 causal, attention alone: S=1024
+  // 30.2 -> 22.2 us, S=2048 40.8 -> 33.6 us.
+  constexpr int NB = 16;  // quads in flight
+  float a0 = 0.f, a1 = 0.f;
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    const f32x4_t v = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(other, (q * 256 + tid) * 16, 0, SC1));
+  for (int b0 = 0; b0 < NQ; b0 += NB) {
+    u32x4_t v[NB];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const float r = o[q / 4][(q % 4) * 4 + k];
-      const float x0 = part == 0 ? r : v[k], x1 = part == 0 ? v[k] : r;
-      o[q / 4][(q % 4) * 4 + k] = fmaf(x0, a0, x1 * a1);
+    for (int q = 0; q < NB; ++q) v[q] = __builtin_amdgcn_raw_buffer_load_b128(other, tid * 16, (b0 + q) * 4096, SC1);
+    __builtin_amdgcn_sched_barrier(0);
+    if (b0 == 0) {
+      const float m0 = part == 0 ? m_run : mo, m1 = part == 0 ? mo : m_run;
+      const float m = fmaxf(m0, m1);
+      // rows past S may hold -inf maxima in both halves; they are not stored
+      a0 = m0 == m ? 1.0f : __builtin_amdgcn_exp2f(m0 - m);
+      a1 = m1 == m ? 1.0f : __builtin_amdgcn_exp2f(m1 - m);
+    }
+#pragma unroll
+    for (int q = 0; q < NB; ++q) {
+      const f32x4_t vq = __builtin_bit_cast(f32x4_t, v[q]);
+      const int n = b0 + q;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float r = o[n / 4][(n % 4) * 4 + k];
+        const float x0 = part == 0 ? r : vq[k], x1 = part == 0 ? vq[k] : r;
+        o[n / 4][(n % 4) * 4 + k] = fmaf(x0, a0, x1 * a1);
+      }
     }
   }
   const float l0 = part == 0 ? l_run : lo, l1 = part == 0 ? lo : l_run;
