@@ -50,7 +50,8 @@ extern "C" {
 #define KFMI_PREP_ROPE 2   /* rope:564 ROPE */
 
 /* mode of kfmi_launch_attention_bf16 (rope:668) */
-#define KFMI_MODE_QUERY 0   /* K prepared once, Q norm(+RoPE) in the attention prologue */
+#define KFMI_MODE_QUERY 0   /* K prepared once, Q norm(+RoPE) in the attention prologue
+                               (small grids: with K, into `out`) */
 #define KFMI_MODE_UNFUSED 1 /* Q and K prepared, plain attention */
 #define KFMI_MODE_FULL 2    /* one launch: Q and K norm(+RoPE) inside attention, K per key tile */
 
@@ -195,7 +196,9 @@ int64_t kfmi_attention_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64
 int kfmi_attention_kernel(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t D, int causal, int mode);
 
 /* The launches of launch_attention (rope:661-677): mode QUERY prepares K
- * into kn (K rows only) then runs attention with the fused Q prologue; mode
+ * into kn (K rows only) then runs attention with the fused Q prologue, or, on
+ * grids of few workgroups (unless out overlaps k), prepares Q rows into out in
+ * the same launch and runs attention on them in place; mode
  * UNFUSED prepares Q into qn and K into kn, then runs plain attention; mode
  * FULL is one launch in which attention normalises (and rotates) Q in its
  * prologue and every K tile as it uses it (FUSE_Q and FUSE_K, rope:619-635;

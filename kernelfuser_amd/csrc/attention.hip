@@ -332,6 +332,27 @@ int attention_kernel(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t D, b
   return k != KFMI_KERNEL_AUTO ? k : attention_kernel_by_shape(B, Hq, Hkv, S, D, causal);
 }
 
+// Whether mode 'query' prepares Q with K in its first launch (into `out`, which
+// the attention launch then reads as prepared Q and overwrites, block by block)
+// instead of in the attention prologue.  On a grid of few workgroups the
+// prologue's arithmetic is on the critical path of one wave per SIMD (10k cycles
+// with RoPE at D = 128, 17k at D = 256), while the preparation launch spreads it
+// over every CU; on larger grids the extra pass over Q costs more.  Measured,
+// causal, graph-replayed, prologue against preparation:
+//   RoPE, D = 128:  16 workgroups (Hq=16 S=128) 12.3 vs 10.1 us (hf), 11.6 vs
+//     9.9 (fp32); 64 (Hq=32 S=256) 14.5 vs 13.4, 13.6 vs 13.0; 96: 16.4 vs
+//     15.7, 15.4 vs 15.4; 128: 13.5 vs 13.4, 12.5 vs 12.6;
+//   RoPE, D = 256:  16 (Hq=16 S=128) 19.3 vs 13.6, 18.2 vs 13.4; 128 (B=8)
+//     23.5 vs 20.0, 22.3 vs 19.8; 144: 36.0 vs 30.3; 192: 58.6 vs 59.0;
+//   no RoPE, D = 128: 32 workgroups 10.9 vs 10.4, 10.7 vs 10.3; 64: 12.7 vs
+//     12.8; D = 256: 64 workgroups 16.7 vs 15.7, 16.0 vs 15.5; 96: 30.3 vs 30.9.
+bool query_prepares_q(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t D, bool causal, bool rope) {
+  if (attention_kernel(B, Hq, Hkv, S, D, causal, false) != KFMI_KERNEL_GENERAL) return false;
+  const int64_t wgs = B * Hq * ((S + 127) / 128), cus = device_cus();
+  if (D == 128) return wgs <= (rope ? cus / 4 : cus / 8);
+  return wgs <= (rope ? cus * 5 / 8 : cus / 4);
+}
+
 }  // namespace kfmi
 
 namespace kfmi {

@@ -349,18 +349,27 @@ static int launch_attention_entry(const void *q, const void *k, const void *v, c
   const bool rope = cos != nullptr;
   // V^T is used by the ping-pong kernel when its rows are 16-byte aligned.
   const bool use_vt = vt != nullptr && kfmi::attention_kernel(B, Hq, Hkv, S, D, causal != 0, false) == KFMI_KERNEL_PINGPONG && S % 8 == 0;
+  // Small grids prepare Q with K, into `out`: every attention workgroup reads its
+  // own query rows before any workgroup that shares them writes them (the halves
+  // of a split block meet first).  Not when `out` overlaps k, which a caller may
+  // reuse because it is dead after the preparation.
+  const uintptr_t o0 = (uintptr_t)out, o1 = o0 + (uintptr_t)(2 * B * Hq * S * D);
+  const uintptr_t k0 = (uintptr_t)k, k1 = k0 + (uintptr_t)(2 * B * Hkv * S * D);
+  const bool prep_q = mode == KFMI_MODE_QUERY && (o1 <= k0 || k1 <= o0) &&
+                      kfmi::query_prepares_q(B, Hq, Hkv, S, D, causal != 0, rope);
+  if (prep_q) qn = out;
+  const bool query = mode == KFMI_MODE_QUERY && !prep_q;
   kfmi::RowsArgs r{};
   r.q = (const uint16_t *)q; r.k = (const uint16_t *)k; r.gq = (const uint16_t *)gq; r.gk = (const uint16_t *)gk;
   r.cos = (const uint16_t *)cos; r.sin = (const uint16_t *)sin; r.qn = (uint16_t *)qn; r.kn = (uint16_t *)kn;
   r.B = B; r.Hq = Hq; r.Hkv = Hkv; r.S = S; r.D = D;
-  r.only_k = mode == KFMI_MODE_QUERY; r.rope = rope; r.style = style_of(norm_style); r.eps = eps;
+  r.only_k = query; r.rope = rope; r.style = style_of(norm_style); r.eps = eps;
   if (use_vt) {  // the preparation launch also writes V^T
     r.v = (const uint16_t *)v;
     r.vt = (uint16_t *)vt;
   }
   hipError_t e = kfmi::launch_rows(r, st);
   if (e != hipSuccess) return launch_status(e, "prepare launch");
-  const bool query = mode == KFMI_MODE_QUERY;
   const int pro = !query ? kfmi::PRO_NONE : (rope ? kfmi::PRO_NORM_ROPE : kfmi::PRO_NORM);
   return attention_impl(query ? q : qn, kn, v, use_vt ? vt : nullptr, gq, nullptr, cos, sin, out, nullptr, B, Hq, Hkv, S, D,
                         scale, eps, causal, pro, style_of(norm_style), bm, bn, st, work, work_bytes);

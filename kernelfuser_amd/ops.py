@@ -170,7 +170,8 @@ def launch_attention(inputs, out, *, causal=False, mode="query", bm=64, bn=64, w
     """Preparation + attention launches of the reference launcher (rope:661-677).
 
     ``mode='query'``: K is prepared once into ``kn``; Q's norm (+RoPE) runs in the
-    attention prologue.  ``mode='unfused'``: Q into ``qn`` and K into ``kn``, then
+    attention prologue, or, on grids of few workgroups, with K in the preparation
+    launch (through ``out``).  ``mode='unfused'``: Q into ``qn`` and K into ``kn``, then
     plain attention.  ``mode='full'``: one launch; attention normalises (and
     rotates) Q in its prologue and each K tile as it uses it -- no scratch, same
     values as ``'query'``.  Scratch buffers must be preallocated for the other
@@ -360,7 +361,8 @@ def fused(q, k, v, gq, gk, cos, sin, causal, eps=EPS, scale=None, norm_style="qw
     style here; ``'hf'`` is accepted as its name in this package) is applied to
     both Q and K.  The reference recomputes K's norm+RoPE for every key tile
     inside one kernel; here K is prepared once (one launch) and Q's
-    norm+RoPE runs in the attention prologue -- the same values, since a K row
+    norm+RoPE runs in the attention prologue (or with K, on small grids) -- the
+    same values, since a K row
     prepared once or per tile is the same function of the same inputs.
     Tables may be [S,D], [B,S,D] or [B,1,S,D] (the first broadcast slice is
     used, rope:193-200)."""
@@ -371,11 +373,14 @@ def fused(q, k, v, gq, gk, cos, sin, causal, eps=EPS, scale=None, norm_style="qw
     b, h, s, d = q.shape
     if tuple(cos.shape) != (s, d) or tuple(sin.shape) != (s, d):
         raise ValueError("Expected rotary tables of S rows")
+    if not float(eps) >= 0.0:
+        raise ValueError("eps must be >= 0")
     out, kn = torch.empty_like(q), torch.empty_like(k)
     with torch.cuda.device(q.device):
-        prepare_attention((q, k, v, gq, gk, cos, sin), None, kn, only_k=True, rope=True, norm_style="hf", eps=eps)
-        attention_prefill(q, kn, v, out, gq=gq, cos=cos, sin=sin, causal=causal, fuse_q=True, norm_style="hf",
-                          scale=scale, eps=eps)
+        wp, wb = _work_args(None, q, k.shape[1], causal)
+        _lib.call("kfmi_launch_attention_bf16", ptr(q), ptr(k), ptr(v), ptr(gq), ptr(gk), ptr(cos), ptr(sin), ptr(out),
+                  None, ptr(kn), None, b, h, k.shape[1], s, d, float(d) ** -0.5 if scale is None else float(scale),
+                  float(eps), int(bool(causal)), MODE_QUERY, NORM_STYLES["hf"], 128, 64, wp, wb, stream_of(q))
     return out
 
 

@@ -1,0 +1,71 @@
+"""Mode 'query' on grids of few workgroups prepares Q with K in its first launch,
+into `out`, and attention reads it there: on both sides of each bound (D, with and
+without RoPE) the launch records show which way the call went, and the output is
+that of mode 'unfused' on a scratch buffer of its own, bit for bit, whole."""
+import pytest
+import torch
+
+import oracle
+from helpers import announce
+from kernelfuser_amd import fused, launch_attention, make_inputs
+
+pytestmark = pytest.mark.gpu
+
+# geometry, B, S, RoPE, Q prepared in the first launch (256 CUs)
+CASES = [((16, 8, 128), 1, 1, True, True), ((16, 8, 128), 1, 130, True, True), ((32, 8, 128), 2, 128, True, True),
+         ((32, 8, 128), 1, 257, True, False), ((32, 8, 128), 1, 100, False, True), ((3, 1, 128), 11, 65, False, False),
+         ((8, 4, 256), 1, 33, True, True), ((16, 8, 256), 1, 1270, True, True), ((16, 8, 256), 1, 1290, True, False),
+         ((8, 4, 256), 1, 700, False, True), ((8, 4, 256), 1, 1025, False, False)]
+
+
+def _launch(xs, causal, rope, style, mode, out=None, qn=None):
+    out = torch.full_like(xs.q, float("nan")) if out is None else out
+    kn = torch.empty_like(xs.k)
+    recs = list(launch_attention(xs.reference7, out, causal=causal, mode=mode, rope=rope, qn=qn, kn=kn,
+                                 norm_style=style))
+    return out, kn, recs
+
+
+@pytest.mark.parametrize("geom,b,s,rope,prepared", CASES)
+@pytest.mark.parametrize("style", ["hf", "fp32"])
+def test_query_prepares_q_on_small_grids(gpu, geom, b, s, rope, prepared, style):
+    xs = make_inputs(b, s, geom, 9100 + s, rope=rope).to(gpu)
+    for causal in (True, False):
+        announce(f"query {geom} B={b} S={s} rope={rope} {style} causal={causal}")
+        out, kn, recs = _launch(xs, causal, rope, style, "query")
+        if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+            # the prologue is the attention instance's fourth argument: 0 for prepared Q
+            assert (recs[1]["kernel"].split(", ")[3] == "0") == prepared, recs
+        ref, kref, _ = _launch(xs, causal, rope, style, "unfused", qn=torch.empty_like(xs.q))
+        torch.cuda.synchronize()
+        assert torch.equal(kn, kref)
+        if prepared:
+            assert torch.equal(out, ref)
+        else:  # the prologue's arithmetic, at most an ulp of Q apart
+            assert oracle.attention_gate(out.cpu(), ref.cpu().float())["pass"]
+
+
+@pytest.mark.parametrize("d", [128, 256])
+def test_query_out_may_reuse_q_or_k(gpu, d):
+    """`out` may be q itself, or k (dead after the preparation), as on larger grids."""
+    xs = make_inputs(1, 96, (4, 4, d), 9300).to(gpu)
+    announce(f"query D={d} out = q, out = k")
+    ref, _, _ = _launch(xs, True, True, "hf", "query")
+    torch.cuda.synchronize()
+    for name in ("q", "k"):
+        ys = make_inputs(1, 96, (4, 4, d), 9300).to(gpu)
+        got, _, _ = _launch(ys, True, True, "hf", "query", out=getattr(ys, name))
+        torch.cuda.synchronize()
+        assert oracle.attention_gate(got.cpu(), ref.cpu().float())["pass"], name
+
+
+def test_fused_small_grid_eps_and_scale(gpu):
+    """The older API's explicit eps and scale reach the preparation of Q."""
+    xs = make_inputs(1, 70, (8, 4, 256), 9400, qkv_std=0.02).to(gpu)
+    announce("fused small grid eps=1e-3 scale=0.05")
+    got = fused(xs.q, xs.k, xs.v, xs.gq, xs.gk, xs.cos, xs.sin, True, eps=1e-3, scale=0.05)
+    torch.cuda.synchronize()
+    ref = oracle.oracle_fp32(*(t.cpu() for t in xs.astuple()), True, scale=0.05, eps=1e-3)
+    assert oracle.attention_gate(got.cpu(), ref)["pass"]
+    with pytest.raises(ValueError, match="eps must be >= 0"):
+        fused(xs.q, xs.k, xs.v, xs.gq, xs.gk, xs.cos, xs.sin, True, eps=-1.0)
