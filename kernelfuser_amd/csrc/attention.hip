@@ -445,6 +445,32 @@ int64_t attention_workspace_counter_bytes(int64_t B, int64_t Hq, int64_t Hkv, in
   return SPLIT_COUNTER_BYTES;
 }
 
+namespace {
+
+// Q heads of one GQA group that a workgroup of the general kernel takes (log2):
+// as many as divide the group, up to four at D = 128 and two at D = 256, each
+// with its share of the 128 query rows.  With fewer positions the workgroup
+// stages fewer rotary-table rows (at D = 256 that is what lets it stage them at
+// all), no wave idles while a neighbour runs key blocks past its own diagonal,
+// and the causal grid is finer: Gemma-3-12B B=8 S=512 57.4 -> 53.0 us,
+// Qwen3-8B B=1 S=2048 47.3 -> 46.8, B=8 S=512 not causal 52.3 -> 51.3.  Without
+// tables to stage, grids of up to one workgroup per CU lose 1-2% (eight layers
+// of Qwen3-0.6B S=128 88.8 vs 89.7 us) and keep one head.
+int heads_per_workgroup_log(int64_t G, int64_t D, bool rope, int64_t wgs, int64_t cus) {
+  if (!rope && wgs <= cus) return 0;
+  if (D == 128 && G % 4 == 0) return 2;
+  return G % 2 == 0 ? 1 : 0;
+}
+// Grids of at least this many workgroups per CU list the query blocks of one KV
+// head after the other (longest first within the head), so that the workgroups
+// running at one time share few heads' K and V in each L2; below, all heads'
+// longest blocks come first, for balance.  Qwen3-8B B=32 S=509 (16 per CU) 162
+// -> 152 us, B=29 S=239 not causal 68.6 -> 61.5; Gemma-3-12B B=8 S=512 (2 per
+// CU) would go from 49.9 to 56.5.
+constexpr int64_t HEAD_MAJOR_WGS_PER_CU = 4;
+
+}  // namespace
+
 hipError_t launch_attention(const AttnArgs &a, hipStream_t stream) {
   constexpr double LOG2E = 1.4426950408889634;
   AttnParams p;
@@ -462,10 +488,6 @@ hipError_t launch_attention(const AttnArgs &a, hipStream_t stream) {
   p.S = a.S;
   p.B = (int)a.B; p.Hq = (int)a.Hq; p.Hkv = (int)a.Hkv;
   p.eps = a.eps;
-  p.by_nbh = FastDiv::of((uint32_t)(a.B * a.Hq));
-  p.by_hq = FastDiv::of((uint32_t)a.Hq);
-  p.by_hkv = FastDiv::of((uint32_t)a.Hkv);
-  p.by_g = FastDiv::of((uint32_t)(a.Hq / a.Hkv));
   const bool factored = a.prologue == PRO_FACTORED_READ || a.prologue == PRO_FACTORED_CALC;
   // rope:636 SCALE*log2e; qk:621 D**-.5*log2e (both formed in double, then FP32)
   p.c_scale = (float)((factored ? 1.0 / sqrt((double)a.D) : a.scale) * LOG2E);
@@ -493,7 +515,7 @@ hipError_t launch_attention(const AttnArgs &a, hipStream_t stream) {
     }
   } else {
     const int nbh = p.B * p.Hq;
-    p.xcd_remap = (nbh % 8 == 0 && (p.B * p.Hkv) % 8 == 0) ? 1 : 0;
+    p.xcd_remap = (p.B * p.Hkv) % 8 == 0 ? 1 : 0;
     blocks = p.n_qblocks * nbh;
     SplitPlan pl;
     if (a.work && tun.split != 1 && plan_split(a.B, a.Hq, a.S, a.D, a.causal, device_cus(), pl)) {
@@ -509,11 +531,24 @@ hipError_t launch_attention(const AttnArgs &a, hipStream_t stream) {
         blocks = pl.n_items * nbh;
       }
     }
+    p.hpw_log = a.gk || p.n_items > 0 ? 0 : heads_per_workgroup_log(a.Hq / a.Hkv, a.D, a.prologue == PRO_NORM_ROPE, blocks, device_cus());
+    p.groups = (int)(a.Hq / a.Hkv) >> p.hpw_log;
+    p.units = p.B * p.Hkv * p.groups;
+    if (p.n_items == 0) {
+      const int64_t rows = 128 >> p.hpw_log;
+      p.n_qblocks = (int)((a.S + rows - 1) / rows);
+      blocks = p.n_qblocks * p.units;
+    }
+    p.by_units = FastDiv::of((uint32_t)p.units);
+    p.by_groups = FastDiv::of((uint32_t)p.groups);
+    p.by_hkv = FastDiv::of((uint32_t)a.Hkv);
+    p.by_kv_wgs = FastDiv::of((uint32_t)(p.groups * p.n_qblocks));
+    p.head_major = a.gk == nullptr && p.n_items == 0 && p.xcd_remap && blocks >= HEAD_MAJOR_WGS_PER_CU * device_cus() ? 1 : 0;
     // D = 128, causal, all workgroups resident in one round of two per CU:
-    // pair each CU's long block with a short one (the head stays the same,
-    // as bid and bid + cus map to the same head when cus % nbh == 0)
+    // pair each CU's long block with a short one (the heads stay the same,
+    // as bid and bid + cus map to the same heads when cus % units == 0)
     const int64_t cus = device_cus();
-    if (a.causal && a.D == 128 && p.n_items == 0 && cus % nbh == 0 && blocks > cus && blocks <= 2 * cus)
+    if (a.causal && a.D == 128 && p.n_items == 0 && cus % p.units == 0 && blocks > cus && blocks <= 2 * cus)
       p.slot2 = (int)cus;
   }
   if (tun.clock_stamps) {
@@ -534,7 +569,7 @@ hipError_t launch_attention(const AttnArgs &a, hipStream_t stream) {
   if (kind == KFMI_KERNEL_PINGPONG || kind == KFMI_KERNEL_WIDE)
     launch_log_plan("hpg=%d persistent=%d xcd=%d", p.pp_hpg, p.pp_units > 0 ? 1 : 0, p.xcd_remap);
   else
-    launch_log_plan("split=%d pair=%d xcd=%d", n_split, p.slot2 > 0 ? 1 : 0, p.xcd_remap);
+    launch_log_plan("split=%d pair=%d xcd=%d heads=%d", n_split, p.slot2 > 0 ? 1 : 0, p.xcd_remap, 1 << p.hpw_log);
   return e;
 }
 

@@ -124,7 +124,12 @@ struct AttnParams {
   // slot takes the query blocks shortest first and each CU's pair sums to
   // the same number of key tiles
   int slot2;
-  FastDiv by_nbh, by_hq, by_hkv, by_g;  // general kernel: B*Hq, Hq, Hkv, Hq/Hkv
+  // General kernel: a workgroup takes 2^hpw_log Q heads of one GQA group x
+  // 128 >> hpw_log query rows; `units` such head groups per query block
+  // (B*Hkv*groups), `groups` of them per KV head.
+  // head_major: the query blocks of a KV head are adjacent in the grid.
+  int hpw_log, units, groups, head_major;
+  FastDiv by_units, by_groups, by_hkv, by_kv_wgs;
   float c_scale;  // scale*log2(e); for the factored prologues D^-1/2*log2(e)
   float eps;
   // Split-KV plan of the general kernel (n_items > 0): work item r of the
@@ -324,8 +329,8 @@ __device__ __forceinline__ void lds_read_offsets(int lane, uint32_t (&kra)[8], u
 // applied to the normalised FP32 row before its single rounding, so the MFMA
 // yields scores already in log2 units and cl becomes 1.
 // Rotary table rows staged in LDS by the caller (STAGED; otherwise read from
-// global memory): the lane's chunk 2c+g of cos is at cos + off[c], of sin at
-// sin + off[c]; the copies are waited for at the barrier inside q_prologue.
+// global memory): the lane's chunk 2c+g of cos is at cos + off[c % 8] +
+// 256 * (c / 8), of sin at the same offset from sin; the copies are waited for at the barrier inside q_prologue.
 // STAGED is a template parameter, not a null test of tab.cos, so that the
 // unused global-load path is not compiled in (its loads, though never
 // executed, made the compiler add waits for them).
@@ -370,6 +375,12 @@ __device__ __forceinline__ void q_prologue(const AttnParams &p, int64_t qoff, in
     // waits for one round trip to memory, not two
     constexpr bool TAB = PRO == PRO_NORM_ROPE;
     constexpr bool GAM = PRO == PRO_NORM || PRO == PRO_NORM_ROPE;
+    // D = 256: the staged rows are read where they are used (all of them at once
+    // would take 128 registers); the caller keeps them in LDS until then
+    constexpr bool LAZY = STAGED && D == 256;
+    auto staged = [&](const unsigned char *t, int c) {
+      return *reinterpret_cast<const u32x4_t *>(t + tab.off[c & 7] + (c >> 3) * 256);
+    };
     u32x4_t graw[GAM ? NC : 1], craw[TAB ? NC : 1], sraw[TAB ? NC : 1];
     if constexpr (GAM) {
 #pragma unroll
@@ -401,8 +412,9 @@ __device__ __forceinline__ void q_prologue(const AttnParams &p, int64_t qoff, in
         __syncthreads();
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
-          craw[c] = *reinterpret_cast<const u32x4_t *>(tab.cos + tab.off[c]);
-          sraw[c] = *reinterpret_cast<const u32x4_t *>(tab.sin + tab.off[c]);
+          if constexpr (LAZY) break;
+          craw[c] = staged(tab.cos, c);
+          sraw[c] = staged(tab.sin, c);
         }
         after_tab();
       }
@@ -434,10 +446,10 @@ __device__ __forceinline__ void q_prologue(const AttnParams &p, int64_t qoff, in
         }
         if constexpr (PRO == PRO_NORM_ROPE) {
           float cs1[8], sn1[8], cs2[8], sn2[8];
-          unpack8(craw[c], cs1);
-          unpack8(sraw[c], sn1);
-          unpack8(craw[c2], cs2);
-          unpack8(sraw[c2], sn2);
+          unpack8(LAZY ? staged(tab.cos, c) : craw[c], cs1);
+          unpack8(LAZY ? staged(tab.sin, c) : sraw[c], sn1);
+          unpack8(LAZY ? staged(tab.cos, c2) : craw[c2], cs2);
+          unpack8(LAZY ? staged(tab.sin, c2) : sraw[c2], sn2);
           if constexpr (ST == ST_FP32) {
 #pragma unroll
             for (int j = 0; j < 8; ++j) {

@@ -1,7 +1,7 @@
 #pragma once
 // The general attention kernel (attn_fwd_kernel): any D in {128, 256} and GQA
-// ratio.  One workgroup = 4 waves = 128 query rows of one head, 32 rows a wave;
-// 16 KiB K and V tiles (64 keys at D = 128, 32 at D = 256), one barrier per
+// ratio.  One workgroup = 4 waves = 128 query rows, 32 rows a wave, of one head
+// or shared between two or four heads of a GQA group; 16 KiB K and V tiles (64 keys at D = 128, 32 at D = 256), one barrier per
 // tile.  attn_fwd128.hip and attn_fwd256.hip instantiate it.
 //
 // Each wave is one instruction stream in which every MFMA has its share of the
@@ -75,12 +75,23 @@ __global__ __launch_bounds__(256, (D == 128 ? 2 : 1)) void attn_fwd_kernel(AttnP
   const int lr = lane & 31;  // query row of this lane within the wave
   const int64_t S = p.S;
 
-  // ---- work item: heaviest query blocks (or split halves) first; KV groups
-  // pinned to an XCD ----
-  const int nbh = p.B * p.Hq;
+  // ---- work item: heaviest query blocks (or split halves) first, over all heads
+  // or (head_major) within a KV head's turn; KV heads pinned to an XCD ----
   const int bid = blockIdx.x;
-  const int rank = p.by_nbh.div(bid);
-  const int r = bid - rank * nbh;
+  int rank, kq, hg;
+  if (p.head_major) {
+    const int j = bid >> 3;
+    kq = p.by_kv_wgs.div(j);
+    const int rem = j - kq * (p.groups * p.n_qblocks);
+    rank = p.by_groups.div(rem);
+    hg = rem - rank * p.groups;
+  } else {
+    rank = p.by_units.div(bid);
+    const int r = bid - rank * p.units;
+    const int jj = p.xcd_remap ? r >> 3 : r;
+    kq = p.by_groups.div(jj);
+    hg = jj - kq * p.groups;
+  }
   int qb, t0 = 0, t1 = -1, sid = -1;
   if (D == 256 && p.n_items > 0) {
     qb = p.it_qb[rank];
@@ -88,28 +99,22 @@ __global__ __launch_bounds__(256, (D == 128 ? 2 : 1)) void attn_fwd_kernel(AttnP
     t1 = p.it_t1[rank];
     sid = p.it_sid[rank];
   } else if (CAUSAL && D == 128 && p.slot2 > 0 && bid >= p.slot2) {
-    qb = p.by_nbh.div(bid - p.slot2);
+    qb = p.by_units.div(bid - p.slot2);
   } else {
     qb = CAUSAL ? p.n_qblocks - 1 - rank : rank;
   }
-  const int G = p.Hq / p.Hkv;
-  int b, h;
-  if (p.xcd_remap) {
-    // Workgroups are dispatched round-robin over the 8 XCDs (bid % 8).  Map
-    // KV group kg to XCD kg % 8 so the G query heads that read the same K/V
-    // share one L2.
-    const int xcd = r & 7, jj = r >> 3;
-    const int jg = p.by_g.div(jj);
-    const int kg = xcd + 8 * jg;
-    b = p.by_hkv.div(kg);
-    h = (kg - b * p.Hkv) * G + jj - jg * G;
-  } else {
-    b = p.by_hq.div(r);
-    h = r - b * p.Hq;
-  }
-  const int kvh = p.by_g.div(h);
+  // Head group hg of KV head kg (batch and KV head).  Workgroups are dispatched
+  // round-robin over the 8 XCDs (bid % 8): with xcd_remap KV head kg runs on XCD
+  // kg % 8, so the query heads that read the same K/V share one L2.
+  const int kg = p.xcd_remap ? (bid & 7) + 8 * kq : kq;
+  const int b = p.by_hkv.div(kg), kvh = kg - b * p.Hkv;
+  // this wave's head of the group and its block of 32 rows
+  const int wl = 2 - p.hpw_log;
+  const int rb = w & ((1 << wl) - 1);
+  const int h = (((kvh * p.groups + hg) << p.hpw_log) + (w >> wl));
+  const int rows = BM >> p.hpw_log;  // query rows per head
   const int64_t qoff = ((int64_t)b * p.Hq + h) * S;
-  const int64_t kvoff = ((int64_t)b * p.Hkv + kvh) * S;
+  const int64_t kvoff = (int64_t)kg * S;
 
   const uint32_t head_bytes = (uint32_t)(S * RB);
   const i32x4_t krs = buffer_rsrc(p.k + kvoff * D, head_bytes);
@@ -122,11 +127,11 @@ __global__ __launch_bounds__(256, (D == 128 ? 2 : 1)) void attn_fwd_kernel(AttnP
     vvo[i] = copy_lane_offset<D>(w * LPW + i, lane, true);
   }
 
-  const int q0 = qb * BM + w * 32;
+  const int q0 = qb * rows + rb * 32;
   const int qrow = q0 + lr;
 
   // ---- KV tile range [t0, nT) of this work item, [u0, nUw) of this wave ----
-  const int64_t kv_end = CAUSAL ? ((int64_t)(qb + 1) * BM < S ? (int64_t)(qb + 1) * BM : S) : S;
+  const int64_t kv_end = CAUSAL ? ((int64_t)(qb + 1) * rows < S ? (int64_t)(qb + 1) * rows : S) : S;
   const int nT = t1 >= 0 ? t1 : (int)((kv_end + BN - 1) / BN);
   const int64_t wave_end = CAUSAL ? ((int64_t)q0 + 32 < S ? (int64_t)q0 + 32 : S) : S;
   // the loop runs over blocks u of 32 keys (tile u / SUB): this wave's end, and
@@ -167,31 +172,48 @@ __global__ __launch_bounds__(256, (D == 128 ? 2 : 1)) void attn_fwd_kernel(AttnP
   // ---- Q prologue ----
   bf16x8_t qreg[NC];
   float cl;
-  if constexpr (PRO == PRO_NORM_ROPE && D == 128) {
-    // The rotary-table rows of the wave's 32 positions are first staged in the
-    // K/V buffers (cos in the first 32 KiB, sin in the second) with coalesced
-    // copies (8 per table per wave, the K tiles' chunk swizzle, so kra[c]
-    // addresses the lane's chunks) instead of loads that each touch 32 rows.
-    // Once every wave holds its rows in registers the first K/V copies are
-    // issued; they land while the prologue computes.
-    StagedTables tab;
+  if constexpr (PRO == PRO_NORM_ROPE) {
+    // The rotary-table rows of the workgroup's positions are first staged in K/V
+    // buffers with coalesced copies (the K tiles' chunk swizzle, so kra addresses
+    // the lane's chunks) instead of loads that each touch 32 rows.
     const i32x4_t crs = buffer_rsrc(p.cos, (uint32_t)(S * RB));
     const i32x4_t srs = buffer_rsrc(p.sin, (uint32_t)(S * RB));
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int j = 8 * w + i;  // rows 4j .. 4j+3 of the block
-      const uint32_t voff = copy_lane_offset<D>(j, lane, false) + (uint32_t)(qb * BM * RB);
-      copy16_to_lds(crs, lds0 + j * 1024, voff);
-      copy16_to_lds(srs, lds0 + 32768 + j * 1024, voff);
-    }
-    tab.cos = smem + w * 32 * RB;
-    tab.sin = tab.cos + 32768;
-    tab.off = kra;
-    q_prologue<D, PRO, ST, false, true>(p, qoff, qrow, qrow < S, g, qreg, cl, tab, [&]() {
-      __syncthreads();  // every wave's table reads have completed
+    const int ncp = rows * RB / 4096;  // 1 KiB copies per wave per table
+    auto stage = [&](int cos0, int sin0) {
+      for (int i = 0; i < ncp; ++i) {
+        const int j = ncp * w + i;
+        const uint32_t voff = copy_lane_offset<D>(j, lane, false) + (uint32_t)qb * (uint32_t)(rows * RB);
+        copy16_to_lds(crs, lds0 + cos0 + j * 1024, voff);
+        copy16_to_lds(srs, lds0 + sin0 + j * 1024, voff);
+      }
+      StagedTables tab;
+      tab.cos = smem + cos0 + rb * 32 * RB;
+      tab.sin = smem + sin0 + rb * 32 * RB;
+      tab.off = kra;
+      return tab;
+    };
+    if constexpr (D == 128) {
+      // 128 or 64 positions: in the buffers of the first tiles, whose copies are
+      // issued once every wave holds its rows in registers (they land while the
+      // prologue computes); 32 positions: in V buffer 1, which no first copy
+      // writes.
+      const bool apart = p.hpw_log == 2;
+      const int cos0 = apart ? VRING + TILE : 0;
+      const StagedTables tab = stage(cos0, cos0 + rows * RB);
+      q_prologue<D, PRO, ST, false, true>(p, qoff, qrow, qrow < S, g, qreg, cl, tab, [&]() {
+        if (!apart) __syncthreads();  // every wave's table reads have completed
+        first_copies();
+      });
+    } else if (p.hpw_log == 1) {
+      // 64 positions: cos in K buffers 2 and 3, sin in V buffers 2 and 3
+      const StagedTables tab = stage(2 * TILE, VRING + 2 * TILE);
       first_copies();
-    });
-  } else if constexpr (PRO == PRO_NORM_ROPE || PRO == PRO_NORM) {
+      q_prologue<D, PRO, ST, false, true>(p, qoff, qrow, qrow < S, g, qreg, cl, tab);
+    } else {
+      first_copies();
+      q_prologue<D, PRO, ST>(p, qoff, qrow, qrow < S, g, qreg, cl);
+    }
+  } else if constexpr (PRO == PRO_NORM) {
     first_copies();
     q_prologue<D, PRO, ST>(p, qoff, qrow, qrow < S, g, qreg, cl);
   }
@@ -549,7 +571,7 @@ __global__ __launch_bounds__(256, (D == 128 ? 2 : 1)) void attn_fwd_kernel(AttnP
   unsigned char *tile = smem + w * (32 * RB);
   if (D != 256 || sid < 0) store_packed<D>(tile, p.out + qoff * D, S, q0, lane, words);
   else if constexpr (D == 256)
-    split_finish<D>(p, tile, sid * nbh + (b * p.Hq + h), t0 > 0 ? 1 : 0, qoff, q0, tid, lane, m_run, l_run, o);
+    split_finish<D>(p, tile, sid * (p.B * p.Hq) + (b * p.Hq + h), t0 > 0 ? 1 : 0, qoff, q0, tid, lane, m_run, l_run, o);
   clock_stamp<true>(p.stamps);
 }
 

@@ -1,8 +1,9 @@
 """The general attention kernel at the sizes where its block pipeline can go
 wrong: one to ten 32-key blocks (the K/V rings of two and four tiles wrap, a
 sweep ends on either buffer and either half of a 64-key tile), ragged last
-blocks and rows, waves with no block at all, and both causal modes, for every
-way Q reaches the matrix cores (prepared, normalised, rotated, factored).
+blocks and rows, waves with no block at all, and both causal modes, for one,
+two and four heads per workgroup (GQA ratios 3, 2 and 4) and every way Q
+reaches the matrix cores (prepared, normalised, rotated, factored).
 Whole output against the FP32 oracle; and the exact redo of the same shapes,
 started by one key far above the first block's row maximum."""
 import pytest
@@ -24,13 +25,12 @@ def _expect(xs, causal, rope):
     return oracle.oracle_fp32(q, k, v, gq, gk, cos if rope else None, sin if rope else None, causal)
 
 
-@pytest.mark.parametrize("d", [128, 256])
+@pytest.mark.parametrize("geom", [(3, 1, 128), (4, 2, 128), (8, 2, 128), (3, 1, 256), (4, 2, 256), (8, 2, 256)])
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("path", ["plain", "norm", "rope", "factored"])
-def test_block_counts_whole_output(gpu, d, causal, path):
-    geom = (3, 1, d) if d == 256 else (6, 2, d)
+def test_block_counts_whole_output(gpu, geom, causal, path):
     for s in SIZES:
-        announce(f"general kernel D={d} S={s} causal={causal} {path}")
+        announce(f"general kernel {geom} S={s} causal={causal} {path}")
         xs = make_inputs(2, s, geom, 7000 + s, rope=path != "factored").to(gpu)
         out = torch.full_like(xs.q, float("nan"))
         kn = torch.empty_like(xs.k)
@@ -85,3 +85,21 @@ def test_redo_whole_output(gpu, d, where):
         assert bool(torch.isfinite(got).all())
         # P and O are each rounded to BF16 (2^-9 relative): within 2^-7 of the largest value
         assert float((got - ref).abs().max()) <= 2.0 ** -7 * float(ref.abs().max()), (s, float((got - ref).abs().max()))
+
+
+@pytest.mark.parametrize("geom,b,s", [((8, 2, 128), 64, 257), ((6, 2, 128), 80, 260), ((4, 2, 256), 128, 250)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_head_major_grid_whole_output(gpu, geom, b, s, causal):
+    """Grids of four or more workgroups per CU, which list the query blocks of
+    one KV head after the other."""
+    announce(f"head-major grid {geom} B={b} S={s} causal={causal}")
+    xs = make_inputs(b, s, geom, 7777).to(gpu)
+    out = torch.full_like(xs.q, float("nan"))
+    kn = torch.empty_like(xs.k)
+    prepare_attention(xs.reference7, None, kn, only_k=True, norm_style="fp32")
+    with _lib.tuning(attn_kernel="general"):
+        attention_prefill(xs.q, kn, xs.v, out, gq=xs.gq, cos=xs.cos, sin=xs.sin, causal=causal, norm_style="fp32")
+        grid = [r["grid"] for r in _lib.last_launches()][-1]
+    torch.cuda.synchronize()
+    assert grid >= 1024, grid  # 4 x 256 CUs
+    assert oracle.attention_gate(out.cpu(), _expect(xs, causal, True))["pass"]
