@@ -131,6 +131,8 @@ def _work_args(work, q, hkv, causal):
     one when the shape splits; a tensor is used as given."""
     if work is None:
         b, h, s, d = q.shape
+        if d == 128 or not causal:  # such shapes never split
+            return None, 0
         work = _workspace(q.device, attention_workspace_bytes(b, h, hkv, s, d, causal))
     if work is None:
         return None, 0
@@ -286,10 +288,27 @@ def _bn(bn):
 # Validated, allocating API
 # ---------------------------------------------------------------------------
 
+class _on_device:
+    """``with torch.cuda.device(device)``, which costs 1.3 us, only when another
+    device is current."""
+
+    def __init__(self, device):
+        index = device.index
+        self.guard = None if index is None or torch.cuda.current_device() == index else torch.cuda.device(device)
+
+    def __enter__(self):
+        if self.guard is not None:
+            self.guard.__enter__()
+
+    def __exit__(self, *exc):
+        return self.guard.__exit__(*exc) if self.guard is not None else False
+
+
 def _check_device(tensors, device):
-    if any((not t.is_cuda) or t.device != device or t.dtype != torch.bfloat16 or not t.is_contiguous()
-           for t in tensors):
-        raise ValueError("Inputs must be contiguous BF16 tensors on one GPU device")
+    bf16 = torch.bfloat16
+    for t in tensors:
+        if not t.is_cuda or t.device != device or t.dtype != bf16 or not t.is_contiguous():
+            raise ValueError("Inputs must be contiguous BF16 tensors on one GPU device")
     if not device_arch(device).startswith("gfx950"):
         raise ValueError(f"This implementation targets gfx950 (MI355X); device is {device_arch(device)}")
 
@@ -376,7 +395,7 @@ def fused(q, k, v, gq, gk, cos, sin, causal, eps=EPS, scale=None, norm_style="qw
     if not float(eps) >= 0.0:
         raise ValueError("eps must be >= 0")
     out, kn = torch.empty_like(q), torch.empty_like(k)
-    with torch.cuda.device(q.device):
+    with _on_device(q.device):
         wp, wb = _work_args(None, q, k.shape[1], causal)
         _lib.call("kfmi_launch_attention_bf16", ptr(q), ptr(k), ptr(v), ptr(gq), ptr(gk), ptr(cos), ptr(sin), ptr(out),
                   None, ptr(kn), None, b, h, k.shape[1], s, d, float(d) ** -0.5 if scale is None else float(scale),
@@ -389,7 +408,7 @@ def anchor(q, k, v, cos, sin, causal, scale=None):
     rope:205-208); the tables are unused."""
     _fused_checks(q, k, v, None, None, None, None)
     out = torch.empty_like(q)
-    with torch.cuda.device(q.device):
+    with _on_device(q.device):
         attention_prefill(q, k, v, out, causal=causal, fuse_q=False, scale=scale)
     return out
 
@@ -402,7 +421,7 @@ def separate(q, k, v, gq, gk, cos, sin, causal, eps=EPS, scale=None, norm_style=
     cos, sin = _position_table(cos, q), _position_table(sin, q)
     _fused_checks(q, k, v, gq, gk, cos, sin)
     qn, kn = torch.empty_like(q), torch.empty_like(k)
-    with torch.cuda.device(q.device):
+    with _on_device(q.device):
         prepare_attention((q, k, v, gq, gk, cos, sin), qn, kn, only_k=False, rope=True, norm_style="hf", eps=eps)
     return anchor(qn, kn, v, cos, sin, causal, scale)
 
@@ -470,7 +489,7 @@ def _optimized_attention_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g
     qn = torch.empty_like(q) if mode == "unfused" else None
     rotary = cos is not None
     xs = (q, k, v, gq, gk, cos if rotary else q, sin if rotary else k)
-    with torch.cuda.device(q.device):
+    with _on_device(q.device):
         launch_attention(xs, out, causal=causal, mode=mode, bm=128, bn=bn, rope=rotary, qn=qn, kn=kn,
                          norm_style=norm_style)
     return out
@@ -495,7 +514,7 @@ def _norm_rope_op(q: torch.Tensor, k: torch.Tensor, gq: torch.Tensor, gk: torch.
                   norm_style: str) -> tuple[torch.Tensor, torch.Tensor]:
     qn = torch.empty_like(q)
     kn = torch.empty_like(k)
-    with torch.cuda.device(q.device):
+    with _on_device(q.device):
         _norm_rope_into(q, k, gq, gk, cos, sin, qn, kn, norm_style)
     return qn, kn
 
@@ -511,7 +530,7 @@ def _factored_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gq: torch.Te
     out = torch.empty_like(q)
     kn = torch.empty_like(k)
     inv = torch.empty(q.shape[:-1], device=q.device, dtype=torch.float32)
-    with torch.cuda.device(q.device):
+    with _on_device(q.device):
         launch_factored_attention((q, k, v, gq, gk), out, inv, kn, causal=causal, bm=128, bn=64)
     return out, inv, kn
 
