@@ -276,35 +276,38 @@ int pp_heads_for(int64_t Hq, int64_t Hkv) {
 
 }  // namespace
 
-// Kernel choice by shape, from the tuning runner's measurements on MI355X
-// (every alternative gated and timed per shape).  The ping-pong kernel needs
-// D = 128 and an even GQA ratio and runs one 512-thread workgroup per CU;
-// below 16 query blocks of 128 rows its per-item Q prologues and few items
-// per CU lose to the general kernel (two 4-wave workgroups per CU): B=1
-// S=1024 27 vs 33 us, B=8 S=1024 causal 100 vs 99 us (FP32 style) and 109
-// vs 105 us (HF style), B=16 S=1024 within 2% either way by style.  The exception is a causal grid
-// whose persistent pairs give every CU exactly one (long, short) unit: B=4
-// S=1000 runs 51.4-53.1 vs 53.8-54.8 us in the FP32 style (paired ratio
-// 1.03-1.04, CI above 1) and ties at 56.5-56.8 us in the HF style.  Units of
-// a few tiles do not pay for their items' prologues: B=32 S=128 (one unit
-// of 3 tiles per CU) runs 37.7 vs 35.6 us, so the exception needs 8 query
-// blocks of 128 rows.  From 16 blocks on
-// it wins when its items fill whole rounds of CUs: non-causal, when the item
-// count is a multiple of the CU count (S=2048 74.8 vs 78.4 us; S=3072, 1.5
-// rounds, 169 vs 156 us for the general kernel); causal, when the persistent
-// pairing applies (Qwen3-32B S=2048 78 vs 83 us; Qwen3-8B S=2048, half the
-// CUs paired, 61.5 vs 54.2 us) and always from 24 blocks (S=3072 93.7 vs
-// 97.2 us, S=4096 141 vs 153 us).  The wide kernel runs only when the
-// tuning overrides ask for it: one wave per SIMD issues the softmax's VALU
-// work and the MFMA stream by itself, and it measures 5-12% slower than the
-// ping-pong kernel from S=3072 on.
+// Kernel choice by shape, from measurements on MI355X (both sides timed in
+// turn, mode 'query', FP32 / HF style).  The ping-pong kernel needs D = 128 and
+// an even GQA ratio and runs one 512-thread workgroup per CU; the general
+// kernel's two 4-wave workgroups per CU hide each other's Q prologues, so the
+// ping-pong kernel is ahead only where its items fill whole rounds of CUs:
+// - below 16 query blocks of 128 rows the general kernel runs (B=8 S=1024 95.9 /
+//   99.4 vs 97.1 / 102.2 us, B=4 S=1536 94.3 / 96.9 vs 98.2 / 102.9), except
+//   causal grids whose persistent pairs give every CU exactly one (long, short)
+//   unit (B=4 S=1000 52.2 / 52.8 vs 51.7 / 53.6) of enough tiles to pay for
+//   their prologues: B=32 S=128 (one unit of 3 tiles per CU) ran 35.6 vs 37.7
+//   us, so at least 8 blocks;
+// - from 16 blocks on, non-causal: when the item count is a multiple of the CU
+//   count (S=2048 69.6 / 70.6 vs 68.8 / 71.8 us, S=8192 902 / 901 vs 865 / 900);
+//   S=3072, 1.5 rounds, 144 / 146 vs 155 / 163;
+// - causal: when the persistent pairing applies (S=4096 136.6 / 138.2 vs 129.8 /
+//   135.2 us, Qwen3-0.6B S=8192 256.7 / 257.1 vs 238.4 / 246.6; Qwen3-8B S=2048,
+//   half the CUs paired, 47.4 / 47.4 vs 55.4 / 57.4), and from 24 blocks also
+//   with more items than CUs (S=3072, 1.5 items per CU, 84.4 / 85.6 vs 86.1 /
+//   89.5).  With at most one item per CU nothing fills the CU when a short item
+//   ends and the longest one sets the time: Qwen3-0.6B S=3072 (192 items) 59.5 /
+//   60.4 vs 71.8 / 75.8 us, S=4096 (256 items) 83.7 / 84.0 vs 97.2 / 101.4; heads
+//   in plain order (Hq=8 Hkv=2 S=8000) 147 / 148 vs 172 / 180.
+// The wide kernel runs only when the tuning overrides ask for it: one wave per
+// SIMD issues the softmax's VALU work and the MFMA stream by itself, and it
+// measures 5-12% slower than the ping-pong kernel from S=3072 on.
 int attention_kernel_by_shape(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t D, bool causal) {
   const int64_t G = Hq / Hkv;
   const int64_t qb128 = (S + 127) / 128;
   if (D != 128 || G % 2 != 0) return KFMI_KERNEL_GENERAL;
-  if (causal && qb128 >= 24) return KFMI_KERNEL_PINGPONG;
   const int64_t cus = device_cus();
   const PpGrid g = pp_grid(B, Hq, Hkv, S, causal, pp_heads_for(Hq, Hkv), cus);
+  if (causal && qb128 >= 24) return g.items > cus ? KFMI_KERNEL_PINGPONG : KFMI_KERNEL_GENERAL;
   const bool paired = causal && g.persistent && thread_tuning().persistent != 1;
   if (qb128 < 16) return paired && g.units == cus && qb128 >= 8 ? KFMI_KERNEL_PINGPONG : KFMI_KERNEL_GENERAL;
   const bool fills = causal ? paired : g.items % cus == 0;
