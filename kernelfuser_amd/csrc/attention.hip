@@ -293,11 +293,12 @@ int pp_heads_for(int64_t Hq, int64_t Hkv) {
 // - causal: when the persistent pairing applies (S=4096 136.6 / 138.2 vs 129.8 /
 //   135.2 us, Qwen3-0.6B S=8192 256.7 / 257.1 vs 238.4 / 246.6; Qwen3-8B S=2048,
 //   half the CUs paired, 47.4 / 47.4 vs 55.4 / 57.4), and from 24 blocks also
-//   with more items than CUs (S=3072, 1.5 items per CU, 84.4 / 85.6 vs 86.1 /
-//   89.5).  With at most one item per CU nothing fills the CU when a short item
-//   ends and the longest one sets the time: Qwen3-0.6B S=3072 (192 items) 59.5 /
-//   60.4 vs 71.8 / 75.8 us, S=4096 (256 items) 83.7 / 84.0 vs 97.2 / 101.4; heads
-//   in plain order (Hq=8 Hkv=2 S=8000) 147 / 148 vs 172 / 180.
+//   with 1.5 items per CU or more (S=3072, just 1.5: 84.4 / 85.6 vs 86.1 / 89.5).
+//   With fewer, little fills a CU whose short item has ended and the longest
+//   items set the time: Qwen3-0.6B S=3072 (192 items on 256 CUs) 59.5 / 60.4 vs
+//   71.8 / 75.8 us, S=4096 (256) 83.7 / 84.0 vs 97.2 / 101.4, S=4500 (288) 100.9 /
+//   101.2 vs 112.2 / 117.0; Hq=16 Hkv=4 S=5000 (316) 117.1 / 117.9 vs 126.2 /
+//   131.6; heads in plain order (Hq=8 Hkv=2 S=8000, 250) 147 / 148 vs 172 / 180.
 // The wide kernel runs only when the tuning overrides ask for it: one wave per
 // SIMD issues the softmax's VALU work and the MFMA stream by itself, and it
 // measures 5-12% slower than the ping-pong kernel from S=3072 on.
@@ -307,7 +308,7 @@ int attention_kernel_by_shape(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int
   if (D != 128 || G % 2 != 0) return KFMI_KERNEL_GENERAL;
   const int64_t cus = device_cus();
   const PpGrid g = pp_grid(B, Hq, Hkv, S, causal, pp_heads_for(Hq, Hkv), cus);
-  if (causal && qb128 >= 24) return g.items > cus ? KFMI_KERNEL_PINGPONG : KFMI_KERNEL_GENERAL;
+  if (causal && qb128 >= 24) return 2 * g.items >= 3 * cus ? KFMI_KERNEL_PINGPONG : KFMI_KERNEL_GENERAL;
   const bool paired = causal && g.persistent && thread_tuning().persistent != 1;
   if (qb128 < 16) return paired && g.units == cus && qb128 >= 8 ? KFMI_KERNEL_PINGPONG : KFMI_KERNEL_GENERAL;
   const bool fills = causal ? paired : g.items % cus == 0;

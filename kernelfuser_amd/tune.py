@@ -16,7 +16,7 @@ calling thread's overrides (``kfmi_set_tuning``):
   ratio is even, there are at least 16 query blocks of 128 rows, and either
   its items fill whole rounds of CUs (non-causal: a multiple of the CU
   count; causal: the persistent pairing applies) or, causal, there are at
-  least 24 blocks and more items than CUs; else general;
+  least 24 blocks and 1.5 items per CU; else general;
 * query heads per ping-pong wave group (``-h1``: two heads x 128 rows per
   item, ``-h2``: four heads x 64 rows); by shape: 2 when the ratio is a
   multiple of 4;

@@ -1,5 +1,5 @@
-"""Causal D = 128 grids from 24 query blocks of 128 rows: with no more
-ping-pong items than compute units the general kernel runs."""
+"""Causal D = 128 grids from 24 query blocks of 128 rows: with fewer than 1.5
+ping-pong items per compute unit the general kernel runs."""
 import pytest
 import torch
 
@@ -11,9 +11,11 @@ from kernelfuser_amd import _lib, launch_attention, make_inputs
     (1, 16, 8, 2944, "general"),    # 23 blocks
     (1, 16, 8, 2945, "general"),    # 24 blocks: 192 items on 256 CUs
     (1, 16, 8, 4096, "general"),    # 256 items
-    (1, 16, 8, 4097, "pingpong"),   # 264 items
+    (1, 16, 8, 6016, "general"),    # 376 items
+    (1, 16, 8, 6017, "pingpong"),   # 384 items
     (1, 16, 8, 8192, "pingpong"),   # paired
-    (1, 32, 4, 2945, "pingpong"),   # four heads per item: 47 blocks of 64 rows, 376 items
+    (1, 32, 4, 3008, "general"),    # four heads per item: 47 blocks of 64 rows, 376 items
+    (1, 32, 4, 3009, "pingpong"),   # 48 blocks, 384 items
     (2, 8, 2, 3200, "general"),     # 200 items, heads in plain order
     (1, 8, 2, 8192, "general"),     # 256 items, heads in plain order
 ])
@@ -22,7 +24,8 @@ def test_kernel_choice(b, hq, hkv, s, kernel):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("geom,b,s", [((16, 8, 128), 1, 2945), ((16, 8, 128), 1, 4096), ((8, 2, 128), 2, 3200)])
+@pytest.mark.parametrize("geom,b,s", [((16, 8, 128), 1, 2945), ((16, 8, 128), 1, 6016), ((8, 2, 128), 2, 3200),
+                                      ((32, 4, 128), 1, 3008)])
 @pytest.mark.parametrize("style", ["fp32", "hf"])
 def test_general_kernel_rows(gpu, geom, b, s, style):
     """Two rows of every query block and the last row pass the oracle gate."""
