@@ -845,6 +845,10 @@ __device__ __forceinline__ uint32_t opaque_bits(float x) {
 __device__ __forceinline__ bool not_finite(float x) {
   return (opaque_bits(x) & 0x7f800000u) == 0x7f800000u;  // exponent field all ones: inf or NaN
 }
+// The lean sweep's bound on a lane's share of a row sum: 2^64 or more, inf or
+// NaN.  Below it the sum of a row's shares, its reciprocal and the scaling of
+// one half of a split item to the other's shift stay far inside FP32's range.
+__device__ __forceinline__ bool sum_too_large(float l) { return (opaque_bits(l) & 0x7fffffffu) >= 0x5f800000u; }
 // Any accumulator inf or NaN: the largest magnitude bit pattern is at least
 // the exponent-all-ones pattern.  Integer arithmetic on one accumulator
 // register: a floating-point sum of the values can be NaN (+inf + -inf),

@@ -12,7 +12,7 @@ import torch
 
 import oracle
 from helpers import announce
-from kernelfuser_amd import anchor
+from kernelfuser_amd import _lib, anchor, attention_prefill
 
 pytestmark = pytest.mark.gpu
 
@@ -55,3 +55,35 @@ def test_lean_matches_exact_on_ordinary_inputs(gpu):
     torch.cuda.synchronize()
     m = oracle.attention_gate(out.cpu(), oracle.attention_fp32(q, k, v, True))
     assert m["pass"], m
+
+
+@pytest.mark.parametrize("d", [128, 256])
+@pytest.mark.parametrize("keys", [(40, 44), (40, 41), (40,), (70, 76, 81)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_row_sums_near_overflow(gpu, d, keys, causal):
+    """Spikes 60 to 130 (log2) above the first block's maximum, small values:
+    the row sum reaches 2^128 and more while O stays finite.  Keys 40 and 44 (mod
+    8 below 4, and 4 or above) are summed by different lanes, so at 127.5 both
+    lanes' sums are finite and only their total is not."""
+    s = 150
+    g = torch.Generator().manual_seed(11)
+    v = (torch.rand(1, 2, s, d, generator=g) - 0.5).bfloat16()
+    unit = 8.0 * d ** -0.5 * 1.4426950408889634  # log2 logit of a key whose component along the queries is 1
+    for level in (60.0, 63.5, 64.5, 120.0, 126.5, 127.25, 127.5, 127.75, 128.5, 130.0):
+        q = torch.zeros(1, 4, s, d, dtype=torch.bfloat16)
+        k = torch.zeros(1, 2, s, d, dtype=torch.bfloat16)
+        q[..., 0] = 8.0
+        c0 = torch.tensor(level / unit).bfloat16().float()  # the level to 2^-16, in two components
+        q[..., 1] = 8.0
+        for key in keys:
+            k[:, :, key, 0] = c0
+            k[:, :, key, 1] = level / unit - c0
+        announce(f"row sum near overflow D={d} keys={keys} level={level} causal={causal}")
+        out = torch.empty_like(q, device=gpu)
+        with _lib.tuning(attn_kernel="general"):
+            attention_prefill(q.to(gpu), k.to(gpu), v.to(gpu), out, causal=causal, fuse_q=False)
+        torch.cuda.synchronize()
+        ref = oracle.attention_fp32(q, k, v, causal)
+        err = float((out.cpu().float() - ref).abs().max())
+        # P and the result are each rounded to BF16 (2^-9 relative), |V| <= 0.5
+        assert err <= 2.0 ** -9, (level, err)
