@@ -849,12 +849,13 @@ __device__ __forceinline__ bool not_finite(float x) {
 // NaN.  Below it the sum of a row's shares, its reciprocal and the scaling of
 // one half of a split item to the other's shift stay far inside FP32's range.
 __device__ __forceinline__ bool sum_too_large(float l) { return (opaque_bits(l) & 0x7fffffffu) >= 0x5f800000u; }
-// Any accumulator inf or NaN: the largest magnitude bit pattern is at least
-// the exponent-all-ones pattern.  Integer arithmetic on one accumulator
+// Any accumulator of magnitude LIMIT (a bit pattern) or more, by default inf or
+// NaN: the largest magnitude bit pattern is at least LIMIT, the
+// exponent-all-ones pattern.  Integer arithmetic on one accumulator
 // register: a floating-point sum of the values can be NaN (+inf + -inf),
 // which code built without NaN semantics may assume away, and a class test
 // per value takes a scalar register pair each.
-template <int N>
+template <uint32_t LIMIT = 0x7f800000u, int N>
 __device__ __forceinline__ bool any_not_finite(const f32x16_t (&o)[N]) {
   uint32_t m[2] = {0u, 0u};
 #pragma unroll
@@ -864,7 +865,7 @@ __device__ __forceinline__ bool any_not_finite(const f32x16_t (&o)[N]) {
       const uint32_t a = __float_as_uint(o[n][i]) & 0x7fffffffu;
       m[i & 1] = m[i & 1] > a ? m[i & 1] : a;
     }
-  return (m[0] > m[1] ? m[0] : m[1]) >= 0x7f800000u;
+  return (m[0] > m[1] ? m[0] : m[1]) >= LIMIT;
 }
 
 }  // namespace

@@ -531,11 +531,13 @@ __global__ __launch_bounds__(256, (D == 128 ? 2 : 1)) void attn_fwd_kernel(AttnP
   // A shift per row is exact as long as no row sum comes near overflow (each
   // lane's share below 2^64; a finite share alone would not do, as two of them
   // can add up to inf) and no accumulator overflows; otherwise the workgroup
-  // redoes the item with the exact online softmax.
-  const bool whole = D != 256 || sid < 0;
-  bool bad = whole ? sum_too_large(l_run) : not_finite(l_run);
-  if (whole) bad |= pack_rows(o, __fdiv_rn(1.0f, sum_halves(l_run)), words);
-  else bad |= any_not_finite(o);
+  // redoes the item with the exact online softmax.  The halves of a split item
+  // are added at the larger of their shifts: accumulators below 2^126 leave room
+  // for that, and a half whose factor flushes to zero (shift 126 or more below)
+  // weighs less than 2^-60 of the other.
+  bool bad = sum_too_large(l_run);
+  if (D != 256 || sid < 0) bad |= pack_rows(o, __fdiv_rn(1.0f, sum_halves(l_run)), words);
+  else bad |= any_not_finite<0x7e800000u>(o);
   if (__syncthreads_or(bad)) {
     Softmax<D, BN, CAUSAL> sm;
 #pragma unroll

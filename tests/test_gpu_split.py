@@ -220,3 +220,64 @@ def test_factored_split_matches_unsplit(gpu, geom, b, s):
     assert bool((d_ <= tol).all()), float((d_ / tol).max())
     inv_ref = oracle.rms_inverse(xs.q.float())[..., 0]
     assert torch.equal(inv_s, inv_u) and torch.allclose(inv_s.cpu(), inv_ref, rtol=1e-6, atol=0)
+
+
+@pytest.mark.parametrize("levels", [(127.5, 0.0, 0.0), (0.0, 0.0, 127.5), (100.0, 0.0, 100.0), (127.75, 0.0, 127.75),
+                                    (127.25, 126.5, 126.5), (64.5, 126.5, 126.5), (126.5, 127.0, 127.0)])
+def test_split_merge_of_spiked_halves(gpu, levels):
+    """Keys far (log2) above the first block's maximum in the first half, in the
+    second half's first block, and behind it: each half's sums are relative to
+    its own first block, and the merge must neither overflow nor drop a half
+    whose shift lies far below the other's."""
+    hq, hkv, s, d = 4, 2, 1000, 256
+    n = attention_workspace_bytes(1, hq, hkv, s, d, True)
+    assert n > 0
+    g = torch.Generator().manual_seed(17)
+    v = (torch.rand(1, hkv, s, d, generator=g) - 0.5).bfloat16()
+    q = torch.zeros(1, hq, s, d, dtype=torch.bfloat16)
+    k = torch.zeros(1, hkv, s, d, dtype=torch.bfloat16)
+    q[..., :2] = 8.0
+    unit = 8.0 * d ** -0.5 * 1.4426950408889634
+    first, start, behind = levels
+    # Keys 40 and 44 are in every block's first half.  The last block's 32 tiles
+    # split at tile 16 (key 512), the block before it (28 tiles) at 448.
+    for level, keys in ((first, (40, 44)), (start, range(448, 544)), (behind, (600, 604))):
+        c0 = torch.tensor(level / unit).bfloat16().float()
+        for key in keys:
+            k[:, :, key, 0] = c0
+            k[:, :, key, 1] = level / unit - c0
+    qd, kd, vd = q.to(gpu), k.to(gpu), v.to(gpu)
+    ref = oracle.attention_fp32(q, k, v, True)
+    announce(f"split merge of spiked halves {levels}")
+    for work in (torch.empty(0, dtype=torch.uint8, device=gpu), torch.zeros(n, dtype=torch.uint8, device=gpu)):
+        out = torch.empty_like(qd)
+        attention_prefill(qd, kd, vd, out, causal=True, fuse_q=False, work=work)
+        torch.cuda.synchronize()
+        err = float((out.cpu().float() - ref).abs().max())
+        # P and the result are each rounded to BF16 (2^-9 relative), |V| <= 0.5
+        assert err <= 2.0 ** -9, (len(work), err)
+
+
+def test_split_merge_of_large_values(gpu):
+    """Accumulators of both halves above 2^127, whose sum overflows, while the
+    result is a value of the inputs' size: 2^62 * 2^65."""
+    hq, hkv, s, d = 4, 2, 1000, 256
+    n = attention_workspace_bytes(1, hq, hkv, s, d, True)
+    q = torch.zeros(1, hq, s, d, dtype=torch.bfloat16)
+    k = torch.zeros(1, hkv, s, d, dtype=torch.bfloat16)
+    v = torch.zeros(1, hkv, s, d, dtype=torch.bfloat16)
+    q[..., :2] = 8.0
+    unit = 8.0 * d ** -0.5 * 1.4426950408889634
+    for key in (40, 600):
+        c0 = torch.tensor(62.5 / unit).bfloat16().float()
+        k[:, :, key, 0] = c0
+        k[:, :, key, 1] = 62.5 / unit - c0
+        v[:, :, key] = 2.0 ** 65
+    announce("split merge of large values")
+    out = torch.empty_like(q, device=gpu)
+    attention_prefill(q.to(gpu), k.to(gpu), v.to(gpu), out, causal=True, fuse_q=False,
+                      work=torch.zeros(n, dtype=torch.uint8, device=gpu))
+    torch.cuda.synchronize()
+    ref = oracle.attention_fp32(q, k, v * 2.0 ** -65, True)
+    err = float((out.cpu().float() * 2.0 ** -65 - ref).abs().max())
+    assert err <= 2.0 ** -8, err  # P and the result are each rounded to BF16, values up to 1
