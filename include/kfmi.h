@@ -197,8 +197,9 @@ int kfmi_attention_kernel(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t
 
 /* The launches of launch_attention (rope:661-677): mode QUERY prepares K
  * into kn (K rows only) then runs attention with the fused Q prologue, or, on
- * grids of few workgroups (unless out overlaps k), prepares Q rows into out in
- * the same launch and runs attention on them in place; mode
+ * grids of few workgroups (unless out overlaps an operand other than q itself),
+ * prepares Q rows into out in the same launch and runs attention on them in
+ * place; mode
  * UNFUSED prepares Q into qn and K into kn, then runs plain attention; mode
  * FULL is one launch in which attention normalises (and rotates) Q in its
  * prologue and every K tile as it uses it (FUSE_Q and FUSE_K, rope:619-635;

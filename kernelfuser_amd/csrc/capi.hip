@@ -351,12 +351,18 @@ static int launch_attention_entry(const void *q, const void *k, const void *v, c
   const bool use_vt = vt != nullptr && kfmi::attention_kernel(B, Hq, Hkv, S, D, causal != 0, false) == KFMI_KERNEL_PINGPONG && S % 8 == 0;
   // Small grids prepare Q with K, into `out`: every attention workgroup reads its
   // own query rows before any workgroup that shares them writes them (the halves
-  // of a split block meet first).  Not when `out` overlaps k, which a caller may
-  // reuse because it is dead after the preparation.
-  const uintptr_t o0 = (uintptr_t)out, o1 = o0 + (uintptr_t)(2 * B * Hq * S * D);
-  const uintptr_t k0 = (uintptr_t)k, k1 = k0 + (uintptr_t)(2 * B * Hkv * S * D);
-  const bool prep_q = mode == KFMI_MODE_QUERY && (o1 <= k0 || k1 <= o0) &&
-                      kfmi::query_prepares_q(B, Hq, Hkv, S, D, causal != 0, rope);
+  // of a split block meet first).  Not when `out` overlaps another operand (q
+  // itself is fine, row by row): `out` is then written while that operand is
+  // still read, where the two-pass form writes it only when k and gk are dead
+  // and, on grids of independent heads, each head's own v and kn.
+  const int64_t qb = 2 * B * Hq * S * D, kb = 2 * B * Hkv * S * D, tb = rope ? 2 * S * D : 0;
+  auto apart = [&](const void *x, int64_t bytes) {
+    const uintptr_t o = (uintptr_t)out, a = (uintptr_t)x;
+    return o + (uintptr_t)qb <= a || a + (uintptr_t)bytes <= o;
+  };
+  const bool prep_q = mode == KFMI_MODE_QUERY && kfmi::query_prepares_q(B, Hq, Hkv, S, D, causal != 0, rope) &&
+                      (out == q || apart(q, qb)) && apart(k, kb) && apart(v, kb) && apart(kn, kb) &&
+                      apart(gq, 2 * D) && apart(gk, 2 * D) && apart(cos, tb) && apart(sin, tb);
   if (prep_q) qn = out;
   const bool query = mode == KFMI_MODE_QUERY && !prep_q;
   kfmi::RowsArgs r{};

@@ -59,6 +59,33 @@ def test_query_out_may_reuse_q_or_k(gpu, d):
         assert oracle.attention_gate(got.cpu(), ref.cpu().float())["pass"], name
 
 
+@pytest.mark.parametrize("d", [128, 256])
+@pytest.mark.parametrize("name", ["gk", "v", "kn", "gq", "cos", "sin", "q"])
+def test_query_out_overlapping_an_operand(gpu, d, name):
+    """`out` over gk (dead after the preparation), over each head's own v or kn
+    (equal head counts, one block per head) and, on a grid of one workgroup, over
+    gamma, the tables or shifted q: Q is not prepared in `out` then."""
+    heads, s = (4, 96) if name in ("gk", "v", "kn") else (1, 64)
+    xs = make_inputs(1, s, (heads, heads, d), 9350).to(gpu)
+    announce(f"query D={d} out over {name}")
+    ref, _, recs = _launch(xs, True, True, "hf", "query")
+    prologue = lambda r: r[1]["kernel"].split(", ")[3]
+    assert prologue(recs) == "0"
+    buf = torch.empty(2 * xs.q.numel(), dtype=torch.bfloat16, device=gpu)
+    out = buf[:xs.q.numel()].view_as(xs.q)
+    ops = dict(zip(("q", "k", "v", "gq", "gk", "cos", "sin"), xs.reference7), kn=torch.empty_like(xs.k))
+    shift = {"gk": 5 * d, "gq": 5 * d, "q": 16 * d}.get(name, 0)
+    over = buf[shift:shift + ops[name].numel()].view_as(ops[name])
+    over.copy_(ops[name])
+    ops[name] = over
+    kn = ops.pop("kn")
+    recs = list(launch_attention(tuple(ops.values()), out, causal=True, mode="query", rope=True, kn=kn,
+                                 norm_style="hf"))
+    torch.cuda.synchronize()
+    assert prologue(recs) == "2", recs
+    assert oracle.attention_gate(out.cpu(), ref.cpu().float())["pass"]
+
+
 def test_fused_small_grid_eps_and_scale(gpu):
     """The older API's explicit eps and scale reach the preparation of Q."""
     xs = make_inputs(1, 70, (8, 4, 256), 9400, qkv_std=0.02).to(gpu)
