@@ -87,6 +87,30 @@ def test_redo_whole_output(gpu, d, where):
         assert float((got - ref).abs().max()) <= 2.0 ** -7 * float(ref.abs().max()), (s, float((got - ref).abs().max()))
 
 
+@pytest.mark.parametrize("d", [128, 256])
+@pytest.mark.parametrize("causal", [True, False])
+def test_redo_when_o_is_nan_and_never_inf(gpu, d, causal):
+    """Values of +-2^100 at probabilities of 2^60, in two 16-key steps: O becomes
+    inf and then NaN beside a finite row sum, where the result is finite."""
+    s = 150
+    q = torch.zeros(1, 4, s, d, dtype=torch.bfloat16)
+    k = torch.zeros(1, 2, s, d, dtype=torch.bfloat16)
+    v = torch.zeros(1, 2, s, d, dtype=torch.bfloat16)
+    q[..., 0] = 8.0
+    k[:, :, [40, 60], 0] = 60.0 / (8.0 * d ** -0.5 * 1.4426950408889634)
+    v[:, :, 40], v[:, :, 60] = 2.0 ** 100, -(2.0 ** 100)
+    announce(f"redo on NaN D={d} causal={causal}")
+    out = torch.empty_like(q, device=gpu)
+    with _lib.tuning(attn_kernel="general"):
+        attention_prefill(q.to(gpu), k.to(gpu), v.to(gpu), out, causal=causal, fuse_q=False)
+    torch.cuda.synchronize()
+    want = torch.zeros(s)  # the two keys cancel in every row that sees both
+    if causal:
+        want[40:60] = 1.0
+    got = out.cpu().double() * 2.0 ** -100
+    assert float((got - want.double()[None, None, :, None]).abs().max()) <= 2.0 ** -8
+
+
 @pytest.mark.parametrize("geom,b,s", [((8, 2, 128), 64, 257), ((6, 2, 128), 80, 260), ((4, 2, 256), 128, 250)])
 @pytest.mark.parametrize("causal", [True, False])
 def test_head_major_grid_whole_output(gpu, geom, b, s, causal):
