@@ -300,7 +300,7 @@ __global__ __launch_bounds__(256, (D == 128 ? 2 : 1)) void attn_fwd_kernel(AttnP
   };
 
   float m_run = -INFINITY, nm = 0.f;
-  float ls[2] = {0.f, 0.f}, lsn[2] = {0.f, 0.f};
+  float l_run = 0.f, ls[4];  // this lane's share of the row sum: whole tiles, and the chains of the present one
   f32x16_t sa, sb;
   bf16x8_t pb[2], kop[8];
   float x[16], pe[16];
@@ -340,20 +340,23 @@ __global__ __launch_bounds__(256, (D == 128 ? 2 : 1)) void attn_fwd_kernel(AttnP
   // two slots after its second FMA.  The first FMA comes three MFMAs after the
   // scores' last one; a pack comes after the last GEMM2 MFMA that reads the
   // previous block's operand, and slots before the first that reads its own.
-  // Row sums made before T = NS go to lsn, which the next iteration folds in:
-  // the last iteration of a sweep makes probabilities of a block that is not
-  // there.
+  // A tile's row sum is made in four chains and added to l_run once, after its
+  // last block (SB), as Softmax::step does: a sweep rounds S / BN + 10 times, where
+  // chains over the whole range would round S / 4 times.  The last iteration of
+  // a sweep makes probabilities of a block that is not there: no iteration adds
+  // that tile's sum, or (second block of a tile) they are masked to zero.
   constexpr int FIRST_F = f_slot<D>(0);
   static_assert(FIRST_F >= N1 + 2 && f_slot<D>(1) + 2 >= N1 + NDB, "scores complete; first operand free");
   static_assert(f_slot<D>(7) + 2 < NS + N1 - 2 && f_slot<D>(15) + 2 < NS + N1 + NDB - 2, "packed before use");
-  auto valu = [&](auto TT, const f32x16_t &s) {
-    constexpr int T = decltype(TT)::value;
+  static_assert(f_slot<D>(15) + 2 - NS < f_slot<D>(0) + 2, "a block's sum ends before the next one's begins");
+  auto valu = [&](auto TT, auto sbc, const f32x16_t &s) {
+    constexpr int T = decltype(TT)::value, SB = decltype(sbc)::value;
     static_for<0, 16>([&](auto ee) {
       constexpr int e = decltype(ee)::value, F = f_slot<D>(e);
       if constexpr (T == F + 2) {
-        if constexpr (T >= NS) ls[e & 1] += pe[e];
-        else if constexpr (e < 2) lsn[e] = pe[e];
-        else lsn[e & 1] += pe[e];
+        if constexpr (SB == 0 && e < 4) ls[e] = pe[e];
+        else ls[e & 3] += pe[e];
+        if constexpr (SB == SUB - 1 && e == 15) l_run += (ls[0] + ls[1]) + (ls[2] + ls[3]);
         if constexpr (e % 2 == 1) pack_pair(pb[e / 8], std::integral_constant<int, (e % 8) / 2>{}, pe[e - 1], pe[e]);
       }
       if constexpr (T == F + 1) pe[e] = __builtin_amdgcn_exp2f(x[e]);
@@ -387,10 +390,13 @@ __global__ __launch_bounds__(256, (D == 128 ? 2 : 1)) void attn_fwd_kernel(AttnP
       if constexpr (m == FIRST_F) {
         pin_valu(std::integral_constant<int, m - 1>{});
         pin_valu(std::integral_constant<int, NS + m - 1>{});
-        pin_reg(ls[0]);
-        pin_reg(ls[1]);
+        pin_reg(l_run);
+        if constexpr (!LAST) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) pin_reg(ls[j]);
+        }
         pin_reg(pb[1]);
-        if (u + 1 >= u_mask && u + 1 < nUw) {
+        if (u + 1 >= u_mask && (!LAST || u + 1 < nUw)) {
           mfma_settle(nxt);
           mask(nxt, u + 1);
         }
@@ -405,12 +411,8 @@ __global__ __launch_bounds__(256, (D == 128 ? 2 : 1)) void attn_fwd_kernel(AttnP
         mfma_o<ACC>(o[i % NDB], vop(vlo[i % 8], vhi[i % 8]), pb[i / NDB]);
       }
       // ---- probabilities ----
-      if constexpr (m == 0) {
-        ls[0] += lsn[0];
-        ls[1] += lsn[1];
-      }
-      valu(std::integral_constant<int, NS + m>{}, cur);
-      valu(mm, nxt);
+      valu(std::integral_constant<int, NS + m>{}, sbc, cur);
+      valu(mm, std::integral_constant<int, K1S>{}, nxt);
       // ---- LDS reads ----
       if constexpr (N1 == 16 && m < 8) kop2[m] = kread(K1B, K1S, std::integral_constant<int, 8 + m>{});
       if constexpr (m >= N1 - 8 && m < N1 + N2 - 8) {
@@ -437,8 +439,9 @@ __global__ __launch_bounds__(256, (D == 128 ? 2 : 1)) void attn_fwd_kernel(AttnP
       }
       if constexpr (m == NS - 1) {
         pin_valu(mm);
-        pin_reg(lsn[0]);
-        pin_reg(lsn[1]);
+        pin_reg(l_run);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) pin_reg(ls[j]);
         pin_reg(pb[0]);
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -510,7 +513,7 @@ __global__ __launch_bounds__(256, (D == 128 ? 2 : 1)) void attn_fwd_kernel(AttnP
       for (int i = 0; i < n; ++i) mt[i] = fmaxf(mt[i], mt[i + n]);
     m_run = max_halves(mt[0]) * cl;
     nm = -m_run;
-    static_for<0, NS>([&](auto mm) { valu(mm, sa); });  // what the slots of iteration u0 - 1 would have computed
+    static_for<0, NS>([&](auto mm) { valu(mm, std::integral_constant<int, 0>{}, sa); });  // what the slots of iteration u0 - 1 would have computed
   }
   for (int t = t0;;) {
     tile_step(std::integral_constant<int, 0>{}, t);
@@ -526,7 +529,7 @@ __global__ __launch_bounds__(256, (D == 128 ? 2 : 1)) void attn_fwd_kernel(AttnP
   }
   mfma_settle_acc<ACC>(o);
   wait_copies();  // no copy may land in the buffers from here on
-  float l_run = ls[0] + ls[1];
+  if (SUB == 2 && (nUw & 1)) l_run += (ls[0] + ls[1]) + (ls[2] + ls[3]);  // ended within a tile
   u32x2_t words[D / 8];
   // A shift per row is exact as long as no row sum comes near overflow (each
   // lane's share below 2^64; a finite share alone would not do, as two of them

@@ -87,3 +87,33 @@ def test_row_sums_near_overflow(gpu, d, keys, causal):
         err = float((out.cpu().float() - ref).abs().max())
         # P and the result are each rounded to BF16 (2^-9 relative), |V| <= 0.5
         assert err <= 2.0 ** -9, (level, err)
+
+
+@pytest.mark.parametrize("d", [128, 256])
+def test_row_sums_of_long_rows(gpu, d):
+    """One key of probability 1 and 30187 of 2^-24.4, too small to change 1.0 one by
+    one in FP32.  Summed by tile first they all count; in a chain over a quarter
+    of the keys that starts at 1.0 a quarter of them would be lost, 3.4e-4 of the
+    sum.  The result lies 1.3e-4 below a tie of BF16 rounding, which that crosses."""
+    s, n = 30188, 30187
+    p = 2.0 ** -24.4
+    exact = n * float(torch.tensor(p).bfloat16()) / (1 + n * p)  # P is BF16 in the product, FP32 in the sum
+    want = torch.tensor(exact, dtype=torch.float64).bfloat16().double()
+    lossy = exact * (1 + n * p) / (1 + 0.75 * n * p)
+    tie = float(want) + 0.5 * 2.0 ** -17  # the spacing of BF16 at 2^-9.5
+    assert exact * (1 + 1e-4) < tie < lossy * (1 - 1e-4)
+    unit = 8.0 * d ** -0.5 * 1.4426950408889634
+    q = torch.zeros(1, 1, s, d, dtype=torch.bfloat16, device=gpu)
+    k = torch.zeros_like(q)
+    v = torch.ones_like(q)
+    q[..., :2] = 8.0
+    c0 = torch.tensor(-24.4 / unit).bfloat16().float()
+    k[:, :, 1:, 0] = c0
+    k[:, :, 1:, 1] = -24.4 / unit - c0
+    v[:, :, 0] = 0.0
+    announce(f"long row sums D={d}")
+    out = torch.empty_like(q)
+    with _lib.tuning(attn_kernel="general"):
+        attention_prefill(q, k, v, out, causal=False, fuse_q=False)
+    torch.cuda.synchronize()
+    assert bool((out == want.bfloat16().item()).all()), (out.unique(), want)
