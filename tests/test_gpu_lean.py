@@ -1,8 +1,8 @@
 """The general attention kernel's lean softmax and its exact redo.
 
 After the first KV tile of a work item the kernel takes p = exp2(logit -
-m_run) with no per-tile max; a lane whose tile sum reaches 2^64 makes the
-whole workgroup redo the item with the exact online softmax.  These inputs
+m_run) with no per-tile max; a lane whose share of a row sum reaches 2^64 makes
+the whole workgroup redo the item with the exact online softmax.  These inputs
 put one key's logit so far above the first tile's row max (up to 163 in log2
 units, where exp2 overflows) that only the redo gives finite, correct rows;
 the FP32 oracle (softmax attention on the same prepared Q/K) is the check.
@@ -87,6 +87,34 @@ def test_row_sums_near_overflow(gpu, d, keys, causal):
         err = float((out.cpu().float() - ref).abs().max())
         # P and the result are each rounded to BF16 (2^-9 relative), |V| <= 0.5
         assert err <= 2.0 ** -9, (level, err)
+
+
+def test_first_tile_sets_the_shift(gpu):
+    """D = 128: the shift is the maximum of the first 64 keys.  Of two keys that
+    count, the larger is in the second 32: its probability is 1 exactly and its
+    weight 1 / (1 + 2^-2.05).  Relative to the first 32 keys' maximum it would be
+    BF16(2^2.05) / (1 + 2^2.05), 0.0037 above, on the other side of a rounding tie that lies 0.3
+    spacings off on either side."""
+    s, x = 64, 2.05
+    exact, other = 1 / (1 + 2.0 ** -x), float(torch.tensor(2.0 ** x).bfloat16()) / (1 + 2.0 ** x)
+    want = torch.tensor(exact).bfloat16()
+    assert want != torch.tensor(other).bfloat16()
+    unit = 8.0 * 128 ** -0.5 * 1.4426950408889634
+    q = torch.zeros(1, 2, s, 128, dtype=torch.bfloat16)
+    k = torch.zeros(1, 2, s, 128, dtype=torch.bfloat16)
+    v = torch.zeros(1, 2, s, 128, dtype=torch.bfloat16)
+    q[..., :2] = 8.0
+    level = torch.full((s,), -60.0)
+    level[5], level[50] = 0.0, x
+    c0 = (level / unit).bfloat16()
+    k[..., 0], k[..., 1] = c0, (level / unit - c0.float()).bfloat16()
+    v[:, :, 50] = 1.0
+    announce("shift of the first tile")
+    out = torch.empty_like(q, device=gpu)
+    with _lib.tuning(attn_kernel="general"):
+        attention_prefill(q.to(gpu), k.to(gpu), v.to(gpu), out, causal=False, fuse_q=False)
+    torch.cuda.synchronize()
+    assert bool((out.cpu() == want).all()), (out.unique(), want)
 
 
 @pytest.mark.parametrize("d", [128, 256])
