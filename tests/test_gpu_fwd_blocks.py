@@ -1,11 +1,12 @@
 """The general attention kernel at the sizes where its block pipeline can go
 wrong: one to ten 32-key blocks (the K/V rings of two and four tiles wrap, a
 sweep ends on either buffer and either half of a 64-key tile), ragged last
-blocks and rows, waves with no block at all, and both causal modes, for one,
-two and four heads per workgroup (GQA ratios 3, 2 and 4) and every way Q
-reaches the matrix cores (prepared, normalised, rotated, factored).
-Whole output against the FP32 oracle; and the exact redo of the same shapes,
-started by one key far above the first block's row maximum."""
+blocks and rows, waves with no block at all, and both causal modes, for every
+way Q reaches the matrix cores (prepared, normalised, rotated, factored) and
+one, two and four heads per workgroup (GQA ratios 3, 2 and 4: with RoPE on any
+grid, the other ways on grids of more workgroups than CUs).  The launch record
+says how many heads a workgroup took.  Whole output against the FP32 oracle;
+and the exact redo, started by one key far above the first tile's row maximum."""
 import pytest
 import torch
 
@@ -25,32 +26,63 @@ def _expect(xs, causal, rope):
     return oracle.oracle_fp32(q, k, v, gq, gk, cos if rope else None, sin if rope else None, causal)
 
 
-@pytest.mark.parametrize("geom", [(3, 1, 128), (4, 2, 128), (8, 2, 128), (3, 1, 256), (4, 2, 256), (8, 2, 256)])
+def _heads(geom, path, workgroups):
+    """Heads per workgroup: as many as divide the GQA group, up to four at D = 128
+    and two at D = 256; one without rotary tables on grids of up to 256."""
+    group = geom[0] // geom[1]
+    if path != "rope" and workgroups <= 256:
+        return 1
+    return 4 if geom[2] == 128 and group % 4 == 0 else 2 if group % 2 == 0 else 1
+
+
+def _check(gpu, geom, b, s, causal, path):
+    announce(f"general kernel {geom} B={b} S={s} causal={causal} {path}")
+    xs = make_inputs(b, s, geom, 7000 + s, rope=path != "factored").to(gpu)
+    out = torch.full_like(xs.q, float("nan"))
+    kn = torch.empty_like(xs.k)
+    rope = path in ("plain", "rope")
+    no_split = torch.empty(0, dtype=torch.uint8, device=gpu)
+    with _lib.tuning(attn_kernel="general"):
+        if path == "factored":
+            inv = torch.empty(xs.q.shape[:-1], device=gpu)
+            prepare_factored((xs.q, xs.k, xs.v, xs.gq, xs.gk), inv, kn)
+            factored_attention(xs.q, kn, xs.v, inv, out, causal=causal, work=no_split)
+        else:
+            qn = torch.empty_like(xs.q)
+            prepare_attention(xs.reference7, qn, kn, rope=rope, norm_style="fp32")
+            if path == "plain":
+                attention_prefill(qn, kn, xs.v, out, causal=causal, fuse_q=False, work=no_split)
+            else:
+                attention_prefill(xs.q, kn, xs.v, out, gq=xs.gq, cos=xs.cos if rope else None,
+                                  sin=xs.sin if rope else None, causal=causal, norm_style="fp32", work=no_split)
+        plan = [r["plan"] for r in _lib.last_launches()][-1]
+    torch.cuda.synchronize()
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        heads = _heads(geom, path, b * geom[0] * -(-s // 128))
+        assert f"heads={heads}" in plan.split(), (plan, heads)
+    gate = oracle.attention_gate(out.cpu(), _expect(xs, causal, rope))
+    assert gate["pass"], (s, gate)
+
+
+GEOMS = [(3, 1, 128), (4, 2, 128), (8, 2, 128), (3, 1, 256), (4, 2, 256), (8, 2, 256)]
+
+
+@pytest.mark.parametrize("geom", GEOMS)
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("path", ["plain", "norm", "rope", "factored"])
 def test_block_counts_whole_output(gpu, geom, causal, path):
     for s in SIZES:
-        announce(f"general kernel {geom} S={s} causal={causal} {path}")
-        xs = make_inputs(2, s, geom, 7000 + s, rope=path != "factored").to(gpu)
-        out = torch.full_like(xs.q, float("nan"))
-        kn = torch.empty_like(xs.k)
-        rope = path in ("plain", "rope")
-        with _lib.tuning(attn_kernel="general"):
-            if path == "factored":
-                inv = torch.empty(xs.q.shape[:-1], device=gpu)
-                prepare_factored((xs.q, xs.k, xs.v, xs.gq, xs.gk), inv, kn)
-                factored_attention(xs.q, kn, xs.v, inv, out, causal=causal)
-            else:
-                qn = torch.empty_like(xs.q)
-                prepare_attention(xs.reference7, qn, kn, rope=rope, norm_style="fp32")
-                if path == "plain":
-                    attention_prefill(qn, kn, xs.v, out, causal=causal, fuse_q=False)
-                else:
-                    attention_prefill(xs.q, kn, xs.v, out, gq=xs.gq, cos=xs.cos if rope else None,
-                                      sin=xs.sin if rope else None, causal=causal, norm_style="fp32")
-        torch.cuda.synchronize()
-        gate = oracle.attention_gate(out.cpu(), _expect(xs, causal, rope))
-        assert gate["pass"], (s, gate)
+        _check(gpu, geom, 2, s, causal, path)
+
+
+@pytest.mark.parametrize("geom", [(4, 2, 128), (8, 2, 128), (4, 2, 256), (8, 2, 256)])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("path", ["plain", "norm", "factored"])
+def test_shared_workgroups_whole_output(gpu, geom, causal, path):
+    """Several heads per workgroup without rotary tables: more than one workgroup
+    per CU, ragged rows that leave waves without any."""
+    for s in (1, 33, 65, 129, 161):
+        _check(gpu, geom, 264 // geom[0], s, causal, path)
 
 
 @pytest.mark.parametrize("d", [128, 256])
@@ -85,6 +117,40 @@ def test_redo_whole_output(gpu, d, where):
         assert bool(torch.isfinite(got).all())
         # P and O are each rounded to BF16 (2^-9 relative): within 2^-7 of the largest value
         assert float((got - ref).abs().max()) <= 2.0 ** -7 * float(ref.abs().max()), (s, float((got - ref).abs().max()))
+
+
+@pytest.mark.parametrize("geom", GEOMS)
+@pytest.mark.parametrize("causal", [True, False])
+def test_redo_of_rotated_rows_whole_output(gpu, geom, causal):
+    """The redo behind the fused prologue (Q normalised and rotated in place), with
+    and without a causal mask, for one, two and four heads per workgroup: one key
+    whose logits lie ~150 (log2) above the others', along the queries' first component."""
+    b, s, d = 3, 150, geom[2]
+    xs = make_inputs(b, s, geom, 7600)
+    key = 100
+    xs.q[..., 0] = 4 * d ** 0.5  # after the norm 4 / sqrt(17) * sqrt(d), times gamma
+    xs.cos[:, 0] = 1.0  # and the rotation leaves it in place
+    xs.cos[:, d // 2] = 1.0
+    xs.sin[:, 0] = 0.0
+    xs.sin[:, d // 2] = 0.0
+    xs = xs.to(gpu)
+    kn = torch.empty_like(xs.k)
+    prepare_attention(xs.reference7, None, kn, only_k=True, norm_style="fp32")
+    kn[:, :, key] = 0.0
+    kn[:, :, key, 0] = 110.0
+    announce(f"redo of rotated rows {geom} causal={causal}")
+    out = torch.full_like(xs.q, float("nan"))
+    with _lib.tuning(attn_kernel="general"):
+        attention_prefill(xs.q, kn, xs.v, out, gq=xs.gq, cos=xs.cos, sin=xs.sin, causal=causal, norm_style="fp32")
+        plan = [r["plan"] for r in _lib.last_launches()][-1]
+    torch.cuda.synchronize()
+    assert f"heads={_heads(geom, 'rope', 0)}" in plan.split(), plan
+    q = oracle.norm_rope_fp32(*(t.cpu() for t in (xs.q, xs.gq, xs.cos, xs.sin)))
+    logits = torch.matmul(q.bfloat16().float()[:, :, key:], kn.cpu().float()[:, :, key, :, None].repeat_interleave(
+        geom[0] // geom[1], 1)) * d ** -0.5 * 1.4426950408889634
+    assert float(logits.min()) > 100.0  # far above the redo's bound in every row that sees the key
+    ref = oracle.attention_fp32(q.bfloat16(), kn.cpu(), xs.v.cpu(), causal)
+    assert oracle.attention_gate(out.cpu(), ref)["pass"]
 
 
 @pytest.mark.parametrize("d", [128, 256])
