@@ -1,5 +1,6 @@
 #pragma once
-// The end of a split-KV work item at D = 256 (attention.hip, attn_d256.hip).
+// The end of a split-KV work item at D = 256 (attn_fwd.h, and mode 'full' in
+// attention.hip).
 #include "attn_common.h"
 
 namespace kfmi {

@@ -72,8 +72,10 @@ const kfmi_tuning &thread_tuning();
 // The attention kernel (KFMI_KERNEL_GENERAL / _PINGPONG / _WIDE) that
 // launch_attention runs for this shape under the thread's overrides; `full`
 // is mode 'full' (always the general kernel).
-bool query_prepares_q(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t D, bool causal, bool rope);
 int attention_kernel(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t D, bool causal, bool full);
+// Whether mode 'query' prepares Q with K in its first launch, into `out`
+// (grids of few workgroups of the general kernel).
+bool query_prepares_q(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t D, bool causal, bool rope);
 // Why the thread's overrides cannot run this geometry (NULL: they can).
 const char *attention_tuning_error(int64_t Hq, int64_t Hkv, int64_t D, bool full);
 // Workspace bytes with which launch_attention splits the key range of the

@@ -131,7 +131,7 @@ def _work_args(work, q, hkv, causal):
     one when the shape splits; a tensor is used as given."""
     if work is None:
         b, h, s, d = q.shape
-        if d == 128 or not causal:  # such shapes never split
+        if d == 128 or not causal:  # the library never splits these (plan_split): no query
             return None, 0
         work = _workspace(q.device, attention_workspace_bytes(b, h, hkv, s, d, causal))
     if work is None:
@@ -175,10 +175,13 @@ def launch_attention(inputs, out, *, causal=False, mode="query", bm=64, bn=64, w
     attention prologue, or, on grids of few workgroups, with K in the preparation
     launch (through ``out``).  ``mode='unfused'``: Q into ``qn`` and K into ``kn``, then
     plain attention.  ``mode='full'``: one launch; attention normalises (and
-    rotates) Q in its prologue and each K tile as it uses it -- no scratch, same
-    values as ``'query'``.  Scratch buffers must be preallocated for the other
-    modes (rope:665-672).  Timings must include every launch, as this function
-    issues them.
+    rotates) Q in its prologue and each K tile as it uses it -- no scratch, the
+    same chain of roundings as ``'query'``.  (Where the preparation launch
+    normalises Q, its sum of squares is added in another order than in the
+    attention prologue: a few elements of Q, and of the result, are an ulp
+    apart.)  Scratch buffers must be preallocated for the other modes
+    (rope:665-672).  Timings must include every launch, as this function issues
+    them.
 
     ``vt`` (optional, shaped like V): scratch for V transposed per head.  When
     given and the shape runs the ping-pong kernel (``uses_vt``), the

@@ -7,6 +7,7 @@ import re
 from pathlib import Path
 
 import pytest
+import torch
 
 from kernelfuser_amd import _lib
 
@@ -128,6 +129,26 @@ def test_workspace_bytes_query(lib):
     # a 12-pair plan keeps the same counter region: its partials start where
     # the 64-pair plan's do
     assert f(1, 4, 2, 640, 256, 1) == 4096 + 12 * 2 * 130 * 256 * 4
+
+
+def test_shapes_without_a_workspace_query(lib):
+    """ops asks for no workspace at D = 128 or without a mask: the library plans no
+    split there, at any size, and does at D = 256, causal."""
+    from kernelfuser_amd import ops
+    asked = []
+    sizes = [1, 64, 129, 257, 512, 1024, 1537, 2048, 4096, 8192, 32768]
+    for d, causal in ((128, 1), (128, 0), (256, 0)):
+        for b, hq, hkv in ((1, 1, 1), (1, 4, 2), (1, 8, 4), (2, 16, 8), (1, 32, 8), (16, 16, 8)):
+            assert all(lib.kfmi_attention_workspace_bytes(b, hq, hkv, s, d, causal) == 0 for s in sizes
+                       if b * hq * s * d < 1 << 31)
+    real = ops.attention_workspace_bytes
+    ops.attention_workspace_bytes = lambda *a: asked.append(a) or 0
+    try:
+        for d, causal in ((128, True), (128, False), (256, False), (256, True)):
+            assert ops._work_args(None, torch.empty(1, 8, 2048, d, device="meta"), 4, causal) == (None, 0)
+    finally:
+        ops.attention_workspace_bytes = real
+    assert asked == [(1, 8, 4, 2048, 256, True)]
 
 
 def test_attention_kernel_query(lib):
