@@ -342,19 +342,26 @@ int attention_kernel(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t D, b
 // prologue's arithmetic is on the critical path of one wave per SIMD (10k cycles
 // with RoPE at D = 128, 17k at D = 256), while the preparation launch spreads it
 // over every CU; on larger grids the extra pass over Q costs more.  Measured,
-// causal, graph-replayed, prologue against preparation:
-//   RoPE, D = 128:  16 workgroups (Hq=16 S=128) 12.3 vs 10.1 us (hf), 11.6 vs
-//     9.9 (fp32); 64 (Hq=32 S=256) 14.5 vs 13.4, 13.6 vs 13.0; 96: 16.4 vs
-//     15.7, 15.4 vs 15.4; 128: 13.5 vs 13.4, 12.5 vs 12.6;
-//   RoPE, D = 256:  16 (Hq=16 S=128) 19.3 vs 13.6, 18.2 vs 13.4; 128 (B=8)
-//     23.5 vs 20.0, 22.3 vs 19.8; 144: 36.0 vs 30.3; 192: 58.6 vs 59.0;
-//   no RoPE, D = 128: 32 workgroups 10.9 vs 10.4, 10.7 vs 10.3; 64: 12.7 vs
-//     12.8; D = 256: 64 workgroups 16.7 vs 15.7, 16.0 vs 15.5; 96: 30.3 vs 30.9.
+// graph-replayed, prologue against preparation, hf and fp32 style:
+//   RoPE, D = 128:  16 workgroups (Hq=16 S=128) causal 13.2 vs 11.1 us, 12.6 vs
+//     10.9, not causal 12.8 vs 10.7, 11.9 vs 10.4; 64 (Hq=32 S=256) 14.7 vs 13.7,
+//     14.0 vs 13.7, not causal 14.5 vs 13.4, 13.6 vs 13.1; 128 (S=512) 18.6 vs
+//     18.8, 17.7 vs 18.2, not causal 18.5 vs 18.8, 17.5 vs 18.0;
+//   RoPE, D = 256, causal:  16 (Hq=16 S=128) 19.2 vs 14.1, 17.9 vs 13.9; 128 (B=8)
+//     22.5 vs 20.0, 21.0 vs 19.7; 160 (S=1280) 45.8 vs 44.2, 44.7 vs 43.9;
+//   not causal, whose workgroups are all as long as the longest:  128 (S=1024)
+//     40.3 vs 38.6, 37.9 vs 37.2; 144 (S=1152) 42.4 vs 40.7, 40.9 vs 41.4; 160
+//     46.2 vs 47.2, 44.6 vs 46.0;
+//   no RoPE, D = 128: 32 workgroups causal 11.6 vs 11.0, 11.3 vs 11.0, not causal
+//     11.1 vs 10.7, 10.7 vs 10.6; 64: 13.6 vs 13.5, 13.2 vs 13.4, not causal 13.1
+//     vs 13.1, 12.7 vs 12.9; D = 256: 64 workgroups 27.3 vs 26.0, 26.5 vs 25.7, not
+//     causal 24.3 vs 23.0, 23.3 vs 22.3; 96: 31.4 vs 31.1, 30.0 vs 30.4, not
+//     causal 30.4 vs 30.4, 28.8 vs 29.6.
 bool query_prepares_q(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t D, bool causal, bool rope) {
   if (attention_kernel(B, Hq, Hkv, S, D, causal, false) != KFMI_KERNEL_GENERAL) return false;
   const int64_t wgs = B * Hq * ((S + 127) / 128), cus = device_cus();
   if (D == 128) return wgs <= (rope ? cus / 4 : cus / 8);
-  return wgs <= (rope ? cus * 5 / 8 : cus / 4);
+  return wgs <= (!rope ? cus / 4 : causal ? cus * 5 / 8 : cus / 2);
 }
 
 }  // namespace kfmi

@@ -11,10 +11,11 @@ from kernelfuser_amd import fused, launch_attention, make_inputs
 
 pytestmark = pytest.mark.gpu
 
-# geometry, B, S, RoPE, Q prepared in the first launch (256 CUs)
+# geometry, B, S, RoPE, Q prepared in the first launch (256 CUs; "causal": only then)
 CASES = [((16, 8, 128), 1, 1, True, True), ((16, 8, 128), 1, 130, True, True), ((32, 8, 128), 2, 128, True, True),
          ((32, 8, 128), 1, 257, True, False), ((32, 8, 128), 1, 100, False, True), ((3, 1, 128), 11, 65, False, False),
-         ((8, 4, 256), 1, 33, True, True), ((16, 8, 256), 1, 1270, True, True), ((16, 8, 256), 1, 1290, True, False),
+         ((8, 4, 256), 1, 33, True, True), ((16, 8, 256), 1, 1020, True, True), ((16, 8, 256), 1, 1030, True, "causal"),
+         ((16, 8, 256), 1, 1270, True, "causal"), ((16, 8, 256), 1, 1290, True, False),
          ((8, 4, 256), 1, 700, False, True), ((8, 4, 256), 1, 1025, False, False)]
 
 
@@ -30,8 +31,10 @@ def _launch(xs, causal, rope, style, mode, out=None, qn=None):
 @pytest.mark.parametrize("style", ["hf", "fp32"])
 def test_query_prepares_q_on_small_grids(gpu, geom, b, s, rope, prepared, style):
     xs = make_inputs(b, s, geom, 9100 + s, rope=rope).to(gpu)
+    bound = prepared
     for causal in (True, False):
         announce(f"query {geom} B={b} S={s} rope={rope} {style} causal={causal}")
+        prepared = causal if bound == "causal" else bound
         out, kn, recs = _launch(xs, causal, rope, style, "query")
         if torch.cuda.get_device_properties(0).multi_processor_count == 256:
             # the prologue is the attention instance's fourth argument: 0 for prepared Q
