@@ -57,7 +57,7 @@ extern "C" {
 
 /* attention kernels (kfmi_tuning.attn_kernel, kfmi_launch_info.kernel) */
 #define KFMI_KERNEL_AUTO 0     /* chosen by shape */
-#define KFMI_KERNEL_GENERAL 1  /* attn_fwd_kernel: 4 waves x 32 rows of one head, D 128 or 256 */
+#define KFMI_KERNEL_GENERAL 1  /* attn_fwd_kernel: 4 waves x 32 rows of one, two or four heads, D 128 or 256 */
 #define KFMI_KERNEL_PINGPONG 2 /* attn_pp_kernel: 8 waves, two wave groups alternating MFMA and softmax phases */
 #define KFMI_KERNEL_WIDE 3     /* attn_ww_kernel: 4 waves x 64 rows, four heads of a GQA group per item */
 

@@ -24,6 +24,7 @@ namespace {
 // 4 waves x 32 rows, GEMM1 of tile t+1 issued ahead of the softmax and GEMM2 of
 // tile t, exact online softmax.
 // ---------------------------------------------------------------------------
+// (FK tells it from the other forms in the name that launch records carry.)
 template <int D, int BN, bool CAUSAL, int PRO, int ST, bool FK>
 __global__ __launch_bounds__(256, (D == 128 ? 2 : 1)) void attn_fwd_kernel(AttnParams p) {
   static_assert(FK && (PRO == PRO_NORM || PRO == PRO_NORM_ROPE), "the other forms: attn_fwd.h");
@@ -293,8 +294,15 @@ int pp_heads_for(int64_t Hq, int64_t Hkv) {
 // - causal: when the persistent pairing applies (S=4096 136.6 / 138.2 vs 129.8 /
 //   135.2 us, Qwen3-0.6B S=8192 256.7 / 257.1 vs 238.4 / 246.6; Qwen3-8B S=2048,
 //   half the CUs paired, 47.4 / 47.4 vs 55.4 / 57.4), and from 24 blocks also
-//   with 1.5 items per CU or more (S=3072, just 1.5: 84.4 / 85.6 vs 86.1 / 89.5).
-//   With fewer, little fills a CU whose short item has ended and the longest
+//   with 1.5 items per CU or more.  The ping-pong kernel leads on unpaired grids
+//   of 1.6 to 2 items per CU (S=3328 99.4 / 101.7 vs 97.5 / 100.9, S=3500 109.2 /
+//   110.4 vs 105.0 / 109.0, S=3840 124.7 / 127.1 vs 120.5 / 125.4); at 1.5 it trails
+//   by 2-4% (S=3072 90.2 / 89.8 vs 92.4 / 92.5, Hq=32 Hkv=16 S=2945 84.5 / 86.2 vs
+//   86.5 / 89.7), which the choice published for S=3072 keeps, and on unpaired
+//   grids beyond 2 mostly too, which no rule here tells apart yet (S=4500 161.5 /
+//   162.6 vs 169.9 / 177.4, S=5000 192 / 194 vs 204 / 212, S=7000 355 / 357 vs 354 /
+//   366; B=2 S=3072 156.1 / 156.6 vs 163.9 / 168.4; Hq=64 S=5000 367 / 370 vs 369 /
+//   385).  Below 1.5, little fills a CU whose short item has ended and the longest
 //   items set the time: Qwen3-0.6B S=3072 (192 items on 256 CUs) 59.5 / 60.4 vs
 //   71.8 / 75.8 us, S=4096 (256) 83.7 / 84.0 vs 97.2 / 101.4, S=4500 (288) 100.9 /
 //   101.2 vs 112.2 / 117.0; Hq=16 Hkv=4 S=5000 (316) 117.1 / 117.9 vs 126.2 /

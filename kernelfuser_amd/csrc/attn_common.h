@@ -22,7 +22,8 @@
 //                    the other computes exponentials.  Each K/V tile staged in
 //                    LDS serves every head of the workgroup.
 //   attn_fwd_kernel  any D in {128, 256} and GQA ratio: 4 waves = 128 query
-//                    rows of one head; every wave pipelines GEMM1, softmax and
+//                    rows of one head, or of two or four heads of a GQA group;
+//                    every wave pipelines GEMM1, softmax and
 //                    GEMM2 of consecutive key blocks inside itself
 //                    (attn_fwd.h; mode 'full': attention.hip, phase by phase).
 //   attn_ww_kernel   D=128, Hq/Hkv a multiple of 4, on request only: 4 waves,
@@ -330,7 +331,8 @@ __device__ __forceinline__ void lds_read_offsets(int lane, uint32_t (&kra)[8], u
 // yields scores already in log2 units and cl becomes 1.
 // Rotary table rows staged in LDS by the caller (STAGED; otherwise read from
 // global memory): the lane's chunk 2c+g of cos is at cos + off[c % 8] +
-// 256 * (c / 8), of sin at the same offset from sin; the copies are waited for at the barrier inside q_prologue.
+// 256 * (c / 8), of sin at the same offset from sin; the copies are waited for at
+// the barrier inside q_prologue.
 // STAGED is a template parameter, not a null test of tab.cos, so that the
 // unused global-load path is not compiled in (its loads, though never
 // executed, made the compiler add waits for them).
@@ -358,9 +360,9 @@ __device__ __forceinline__ void q_prologue(const AttnParams &p, int64_t qoff, in
   for (int c = 0; c < NC; ++c) raw[c] = qvalid ? ld16(qbase + (int64_t)qrow * D + 16 * c + 8 * g) : zero;
   if constexpr (PRO == PRO_NONE) {
     // The loaded rows are pinned as computed VGPR values (an empty asm that
-    // rewrites them): left as plain loads, the general kernel's tile loop was
-    // scheduled 28% slower in cycles at D=256 (84 against 66 us, Gemma-3-12B
-    // B=1 S=2048) and 7% slower at D=128, with the same instruction counts.
+    // rewrites them), so that the compiler schedules no tile loop around plain
+    // loads: an earlier general kernel, which took this path, lost 28% of its
+    // cycles that way at D=256 and 7% at D=128 (now the ping-pong kernel's path).
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       qreg[c] = as_bf16x8(raw[c]);

@@ -99,9 +99,9 @@ __device__ __forceinline__ void static_for(F &&f) {
 }
 
 // The Q prologue of q_prologue (attn_common.h) for rows that are not normalised,
-// in two halves, so that a kernel puts other work into the loads' round trip.  Rows at or past S load the last
-// row: every load is unconditional and in bounds, and what those rows compute
-// is never stored.
+// in two halves, so that a kernel puts other work into the loads' round trip.
+// Rows at or past S load the last row: every load is unconditional and in
+// bounds, and what those rows compute is never stored.
 template <int D, int PRO, int ST>
 struct QRows {
   static constexpr int NC = D / 16;
