@@ -174,8 +174,9 @@ int kfmi_attention_bf16(const void *q, const void *k, const void *v, const void 
 
 /* Bytes of the optional split-KV workspace `work` of the attention entry
  * points for this shape (0: the shape never splits; -1: invalid shape).
- * For causal D = 256 shapes with no more query blocks than the GPU has CUs
- * (that kernel runs one workgroup per CU), the key range of the longest
+ * For causal D = 256 shapes with fewer query blocks of 128 rows than the GPU
+ * has CUs (that kernel runs one workgroup per CU) and more than 256 keys, the
+ * key range of the longest
  * query blocks is split over two workgroups whose partial results are merged
  * by the one finishing second; the workspace holds a 4 KiB region of
  * arrival counters (the same for every shape) followed by those partials.

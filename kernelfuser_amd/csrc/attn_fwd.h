@@ -1,8 +1,9 @@
 #pragma once
 // The general attention kernel (attn_fwd_kernel): any D in {128, 256} and GQA
 // ratio.  One workgroup = 4 waves = 128 query rows, 32 rows a wave, of one head
-// or shared between two or four heads of a GQA group; 16 KiB K and V tiles (64 keys at D = 128, 32 at D = 256), one barrier per
-// tile.  attn_fwd128.hip and attn_fwd256.hip instantiate it.
+// or shared between two or four heads of a GQA group; 16 KiB K and V tiles (64
+// keys at D = 128, 32 at D = 256), one barrier per tile.  attn_fwd128.hip and
+// attn_fwd256.hip instantiate it, with NaN semantics (pack_rows).
 //
 // Each wave is one instruction stream in which every MFMA has its share of the
 // other work beside it: iteration u issues GEMM1 of key block u+1 and GEMM2 of
@@ -15,13 +16,14 @@
 // preparation launch) and 1530 for 1024 at D = 128 with two workgroups on the
 // CU, 1830 alone (2.0k before; B=1 S=2048 Hq=32: 49.5 -> 47 us).
 //
-// What bounds it now: with the matrix cores ~70% busy the GPU's power
-// management lowers the clock (2.4 GHz on small grids, 1.6-1.8 GHz on long
-// ones); leaving out the exponentials, the copies, or half of the LDS reads of
-// a D = 256 iteration takes 9%, 11% and 0% off its cycles.  Short sequences
-// are bound by what surrounds the loop: per workgroup and 8 tiles (17k cycles
-// at D = 128) 15-18k cycles of norm + RoPE prologue, 1.5k to the first tile's
-// maximum, 3k of epilogue.
+// What bounds it now: with the loop's matrix cores ~70% busy the GPU's power
+// management lowers the clock (B=2 S=2048 factored 2.34 -> 2.01 GHz, B=1 S=2048
+// at D = 128 1.92); leaving out the exponentials, the copies, or half of the LDS
+// reads of a D = 256 iteration takes 9%, 11% and 0% off its cycles.  Short
+// sequences are bound by what surrounds the loop: per workgroup and 8 tiles
+// (16-18k cycles at D = 128) 13k cycles of norm + RoPE prologue (prepared Q 4.5k),
+// 2.5-3k to the first tile's maximum, 2.7k of epilogue; at D = 256 and 16 tiles
+// (22-23k) 21k (9k), 2-3k and 5k.
 #include <cstdio>
 #include <string>
 #include <type_traits>
