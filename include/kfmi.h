@@ -175,17 +175,17 @@ int kfmi_attention_bf16(const void *q, const void *k, const void *v, const void 
 /* Bytes of the optional split-KV workspace `work` of the attention entry
  * points for this shape (0: the shape never splits; -1: invalid shape).
  * For causal D = 256 shapes with fewer query blocks of 128 rows than the GPU
- * has CUs (that kernel runs one workgroup per CU) and more than 256 keys, the
- * key range of the longest
+ * has CUs (that kernel runs one workgroup per CU), the key range of the longest
  * query blocks is split over two workgroups whose partial results are merged
  * by the one finishing second; the workspace holds a 4 KiB region of
  * arrival counters (the same for every shape) followed by those partials.
  * The caller zero-fills it once when allocating; each launch leaves the
  * counters at zero again, so one workspace serves any sequence of shapes
  * that fit in it.  Calls that share a workspace must not overlap in time.
- * With work == NULL or work_bytes below this size the launch does not split
- * (same results, slower on those shapes).  No counterpart in the reference,
- * whose launches never split a query block. */
+ * Up to 256 keys only mode FULL splits; the other modes leave the workspace
+ * alone there.  With work == NULL or work_bytes below this size the launch
+ * does not split (same results, slower on those shapes).  No counterpart in
+ * the reference, whose launches never split a query block. */
 int64_t kfmi_attention_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t D, int causal);
 
 /* The attention kernel (KFMI_KERNEL_GENERAL, _PINGPONG or _WIDE) that an

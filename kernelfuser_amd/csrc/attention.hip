@@ -387,7 +387,9 @@ namespace {
 // second holds the diagonal), and all items are listed longest first.
 // Measured (attention alone, causal, split against unsplit): Gemma-3-4B S=2048
 // 33.6 vs 45.6 us, S=1024 22.2 vs 26.1, S=512 17.3 vs 16.6; a merge costs about
-// 4.5 us, so blocks of up to 8 key tiles stay whole (S=256 14.2 vs 11.6 us).
+// 4.5 us, so blocks of up to 8 key tiles stay whole (S=256 14.2 vs 11.6 us),
+// except in mode 'full', whose tiles cost several times as much (S=200 Hq=8 71.0
+// vs 51.0 us with RoPE, 39.1 vs 31.8 without).
 // A grid that already fills every CU (Gemma-3-12B S=2048, 256 workgroups) loses
 // by splitting, so the plan needs fewer query blocks than CUs (Gemma-3-12B
 // S=1536, 192 blocks: 36.8 vs 37.8 us).  At D = 128 two workgroups share each
@@ -408,13 +410,13 @@ struct SplitPlan {
   int16_t qb[MAX_SPLIT_ITEMS], t0[MAX_SPLIT_ITEMS], t1[MAX_SPLIT_ITEMS], sid[MAX_SPLIT_ITEMS];
 };
 
-bool plan_split(int64_t B, int64_t Hq, int64_t S, int64_t D, bool causal, int64_t cus, SplitPlan &pl) {
+bool plan_split(int64_t B, int64_t Hq, int64_t S, int64_t D, bool causal, bool full, int64_t cus, SplitPlan &pl) {
   const int64_t BM = 128, BN = D == 128 ? 64 : 32;
   const int64_t nqb = (S + BM - 1) / BM;
   if (D != 256 || !causal || nqb < 2 || B * Hq * nqb >= cus) return false;
   auto tiles = [&](int64_t qb) { return ((qb + 1) * BM < S ? (qb + 1) * BM : S) + BN - 1; };
   const int64_t t_max = tiles(nqb - 1) / BN;
-  if (t_max <= 8) return false;
+  if (t_max <= 8 && !full) return false;
   const int64_t half = (t_max + 1) / 2;
   struct Item { int qb, t0, t1, sid; };
   Item items[MAX_SPLIT_ITEMS];
@@ -451,16 +453,17 @@ int64_t split_partial_bytes(int64_t pairs, int64_t D) { return pairs * 2 * (D / 
 
 }  // namespace
 
-int64_t attention_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t D, bool causal) {
+int64_t attention_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t D, bool causal, bool full) {
   SplitPlan pl;
-  if (!plan_split(B, Hq, S, D, causal, device_cus(), pl)) return 0;
+  if (!plan_split(B, Hq, S, D, causal, full, device_cus(), pl)) return 0;
   const int64_t pairs = (int64_t)pl.n_split * B * Hq;
   return SPLIT_COUNTER_BYTES + split_partial_bytes(pairs, D);
 }
 
-int64_t attention_workspace_counter_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t D, bool causal) {
+int64_t attention_workspace_counter_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t D, bool causal,
+                                          bool full) {
   SplitPlan pl;
-  if (!plan_split(B, Hq, S, D, causal, device_cus(), pl)) return 0;
+  if (!plan_split(B, Hq, S, D, causal, full, device_cus(), pl)) return 0;
   return SPLIT_COUNTER_BYTES;
 }
 
@@ -537,7 +540,7 @@ hipError_t launch_attention(const AttnArgs &a, hipStream_t stream) {
     p.xcd_remap = (p.B * p.Hkv) % 8 == 0 ? 1 : 0;
     blocks = p.n_qblocks * nbh;
     SplitPlan pl;
-    if (a.work && tun.split != 1 && plan_split(a.B, a.Hq, a.S, a.D, a.causal, device_cus(), pl)) {
+    if (a.work && tun.split != 1 && plan_split(a.B, a.Hq, a.S, a.D, a.causal, a.gk != nullptr, device_cus(), pl)) {
       const int64_t pairs = (int64_t)pl.n_split * nbh;
       if (a.work_bytes >= SPLIT_COUNTER_BYTES + split_partial_bytes(pairs, a.D)) {
         n_split = pl.n_split;

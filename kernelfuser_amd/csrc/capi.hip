@@ -255,7 +255,7 @@ static int attention_impl(const void *q, const void *k, const void *v, const voi
 int64_t kfmi_attention_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t D, int causal) {
   if (check_shape(B, Hq, Hkv, S, D) != KFMI_OK) return -1;
   g_error.clear();
-  return kfmi::attention_workspace_bytes(B, Hq, Hkv, S, D, causal != 0);
+  return kfmi::attention_workspace_bytes(B, Hq, Hkv, S, D, causal != 0, true);
 }
 
 int kfmi_attention_kernel(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t D, int causal, int mode) {
@@ -326,14 +326,15 @@ static int launch_attention_entry(const void *q, const void *k, const void *v, c
   if (noalloc) {
     // A plan larger than the static array runs unsplit (no workspace), as
     // kfmi_launch_attention_bf16 does when given none.
-    const int64_t need = kfmi::attention_workspace_bytes(B, Hq, Hkv, S, D, causal != 0);
+    const bool full = mode == KFMI_MODE_FULL;
+    const int64_t need = kfmi::attention_workspace_bytes(B, Hq, Hkv, S, D, causal != 0, full);
     work = nullptr;
     work_bytes = 0;
     if (need > 0 && need <= KFMI_SCRATCH_BYTES) {
       hipError_t e = kfmi::noalloc_scratch(&work);
       if (e != hipSuccess) return launch_status(e, "static scratch address");
       work_bytes = KFMI_SCRATCH_BYTES;
-      clear_bytes = kfmi::attention_workspace_counter_bytes(B, Hq, Hkv, S, D, causal != 0);
+      clear_bytes = kfmi::attention_workspace_counter_bytes(B, Hq, Hkv, S, D, causal != 0, full);
     }
   }
   hipStream_t st = (hipStream_t)stream;

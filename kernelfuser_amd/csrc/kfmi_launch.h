@@ -79,11 +79,13 @@ bool query_prepares_q(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t D, 
 // Why the thread's overrides cannot run this geometry (NULL: they can).
 const char *attention_tuning_error(int64_t Hq, int64_t Hkv, int64_t D, bool full);
 // Workspace bytes with which launch_attention splits the key range of the
-// longest causal query blocks over two workgroups (0: this shape never splits).
-int64_t attention_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t D, bool causal);
+// longest causal query blocks over two workgroups (0: this shape never splits);
+// `full` is mode 'full', which splits wherever another mode does.
+int64_t attention_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t D, bool causal, bool full);
 // Leading bytes of that workspace that hold the arrival counters, which must
 // be zero when a launch starts (0: this shape never splits).
-int64_t attention_workspace_counter_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t D, bool causal);
+int64_t attention_workspace_counter_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t S, int64_t D, bool causal,
+                                          bool full);
 
 // Static split-KV workspace of the allocation-free entry point (one per GPU):
 // 36 MiB covers every causal D = 256 split plan of up to 141 (block, head)

@@ -92,7 +92,8 @@ _work_bytes_cache: dict[tuple, int] = {}
 def attention_workspace_bytes(b: int, hq: int, hkv: int, s: int, d: int, causal: bool) -> int:
     """Workspace bytes with which attention splits the longest causal query
     blocks over two workgroups for this shape on the current device (0: it
-    never splits).  Cached per (device, shape)."""
+    never splits; up to 256 keys only mode 'full' does).  Cached per (device,
+    shape)."""
     key = (torch.cuda.current_device() if torch.cuda.is_available() else -1, b, hq, hkv, s, d, bool(causal))
     n = _work_bytes_cache.get(key)
     if n is None:
@@ -126,12 +127,13 @@ def _workspace(device: torch.device, nbytes: int):
     return buf
 
 
-def _work_args(work, q, hkv, causal):
+def _work_args(work, q, hkv, causal, full=False):
     """(pointer, bytes) of the split workspace: ``work=None`` uses the cached
     one when the shape splits; a tensor is used as given."""
     if work is None:
         b, h, s, d = q.shape
-        if d == 128 or not causal:  # the library never splits these (plan_split): no query
+        # the library never splits these (plan_split; up to 256 keys mode 'full' does): no query
+        if d == 128 or not causal or (s <= 256 and not full):
             return None, 0
         work = _workspace(q.device, attention_workspace_bytes(b, h, hkv, s, d, causal))
     if work is None:
@@ -207,7 +209,7 @@ def launch_attention(inputs, out, *, causal=False, mode="query", bm=64, bn=64, w
         raise ValueError("Missing scratch buffers")
     q, k, v, gq, gk, cos, sin = inputs
     b, h, s, d = q.shape
-    wp, wb = _work_args(work, q, k.shape[1], causal)
+    wp, wb = _work_args(work, q, k.shape[1], causal, mode == "full")
     _lib.call("kfmi_launch_attention_bf16",
               ptr(q), ptr(k), ptr(v), ptr(gq), ptr(gk),
               ptr(cos) if rope else None, ptr(sin) if rope else None,

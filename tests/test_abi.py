@@ -132,8 +132,9 @@ def test_workspace_bytes_query(lib):
 
 
 def test_shapes_without_a_workspace_query(lib):
-    """ops asks for no workspace at D = 128 or without a mask: the library plans no
-    split there, at any size, and does at D = 256, causal."""
+    """ops asks for no workspace at D = 128 or without a mask, where the library
+    plans no split at any size, nor up to 256 keys except in mode 'full' (the GPU
+    tests read the launch plans there)."""
     from kernelfuser_amd import ops
     asked = []
     sizes = [1, 64, 129, 257, 512, 1024, 1537, 2048, 4096, 8192, 32768]
@@ -146,9 +147,11 @@ def test_shapes_without_a_workspace_query(lib):
     try:
         for d, causal in ((128, True), (128, False), (256, False), (256, True)):
             assert ops._work_args(None, torch.empty(1, 8, 2048, d, device="meta"), 4, causal) == (None, 0)
+        for s, full in ((256, False), (257, False), (256, True)):
+            ops._work_args(None, torch.empty(1, 8, s, 256, device="meta"), 4, True, full)
     finally:
         ops.attention_workspace_bytes = real
-    assert asked == [(1, 8, 4, 2048, 256, True)]
+    assert asked == [(1, 8, 4, s, 256, True) for s in (2048, 257, 256)]
 
 
 def test_attention_kernel_query(lib):

@@ -13,7 +13,8 @@ import torch
 
 import oracle
 from helpers import announce, bf16_ulp
-from kernelfuser_amd import attention_prefill, attention_workspace_bytes, make_inputs, prepare_attention
+from kernelfuser_amd import (attention_prefill, attention_workspace_bytes, launch_attention, make_inputs,
+                             prepare_attention)
 
 pytestmark = pytest.mark.gpu
 
@@ -281,3 +282,24 @@ def test_split_merge_of_large_values(gpu):
     ref = oracle.attention_fp32(q, k, v * 2.0 ** -65, True)
     err = float((out.cpu().float() * 2.0 ** -65 - ref).abs().max())
     assert err <= 2.0 ** -8, err  # P and the result are each rounded to BF16, values up to 1
+
+
+@pytest.mark.parametrize("s", [129, 200, 256, 257])
+def test_short_blocks_split_in_mode_full_only(gpu, s):
+    """Up to 256 keys a split pays in mode 'full' alone; the other modes leave a
+    workspace alone there, and every mode splits beyond."""
+    geom = (8, 4, 256)
+    xs = make_inputs(1, s, geom, 2323).to(gpu)
+    ref = oracle.oracle_fp32(*(t.cpu() for t in xs.astuple()), True)
+    nbytes = attention_workspace_bytes(1, *geom[:2], s, 256, True)
+    assert nbytes > 0
+    for mode in ("full", "query", "unfused"):
+        for work in (None, torch.zeros(nbytes, dtype=torch.uint8, device=gpu)):
+            announce(f"short split S={s} {mode} workspace={work is not None}")
+            out, kn, qn = torch.empty_like(xs.q), torch.empty_like(xs.k), torch.empty_like(xs.q)
+            recs = list(launch_attention(xs.reference7, out, causal=True, mode=mode, kn=kn, qn=qn, norm_style="fp32",
+                                         work=work))
+            torch.cuda.synchronize()
+            assert recs[-1]["plan"].startswith("split=0") == (mode != "full" and s <= 256), recs[-1]
+            assert oracle.attention_gate(out.cpu(), ref)["pass"]
+            assert work is None or int(work[:4096].count_nonzero()) == 0
