@@ -170,10 +170,13 @@ __global__ __launch_bounds__(256, (D == 128 ? 2 : 1)) void attn_fwd_kernel(AttnP
   wait_copies();
   __syncthreads();
   if (t0 < nTw) gemm1_fused_k<D, BN, ST, PRO == PRO_NORM_ROPE>(smem, K0, kra, qreg, sa, p, t0 * BN, g, lr);
-  for (int t = t0; t < nT;) {
-    iteration(std::integral_constant<int, 0>{}, t, sa, sb);
-    if (++t >= nT) break;
+  // the first iteration stands by itself: with it in the loop D = 256 ran 1-3%
+  // slower (S=1024 171.0 vs 166.8 us, S=200 51.0 vs 47.2, Hq=16 and 8, RoPE)
+  iteration(std::integral_constant<int, 0>{}, t0, sa, sb);
+  for (int t = t0 + 1; t < nT;) {
     iteration(std::integral_constant<int, 1>{}, t, sb, sa);
+    if (++t >= nT) break;
+    iteration(std::integral_constant<int, 0>{}, t, sa, sb);
     ++t;
   }
 
